@@ -108,6 +108,20 @@ __device__ __forceinline__ int sk_even_weight(const MqParams& p) {
   return p.cu_q == nullptr ? kSkEvenWeight : kSkPairWeight / 2;
 }
 
+// Workgroups that take stages.  Every one of them gets two stages or more, so
+// no range is empty (a weighted share is at least 31/32 of the mean) and
+// every workgroup between a cut pair's first and last owner left a partial.
+// A call too small to give the whole grid four stages each uses half of the
+// grid at most: what such a call costs is the chain load -> partial -> merge,
+// and a stage more per workgroup costs it less than twice the contributors
+// (one sequence on 8 kv heads, us per call, at least 1 / 2 / 4 stages each:
+// 64 tokens 10.2 / 11.1 / 11.9, 777 tokens 12.4 / 12.4 / 14.0, 2,048 tokens
+// 13.4 / 13.3 / 14.5, 8,192 tokens 17.9 / 17.8 / 16.6).
+__device__ __forceinline__ int sk_active_wgs(const MqParams& p, int64_t T) {
+  const int64_t n = max(min(T / 2, (int64_t)p.sk_wgs / 2), T / 4);
+  return (int)max((int64_t)1, min((int64_t)p.sk_wgs, n));
+}
+
 // C(w) in the integer type U (uint32_t when T * C(W) + T < 2^32, see
 // sk_fits32, else uint64_t: a 64-bit division is a long instruction
 // sequence, so each caller picks the type once and does all its range
@@ -174,8 +188,8 @@ __device__ __forceinline__ void sk_merge_one(const MqParams& p, int b, int idx, 
     out[lane] = 0u;
     return;
   }
-  const int W = p.sk_wgs;
   const int64_t T = (int64_t)NHG * p.sk_prefix[p.num_seqs];
+  const int W = sk_active_wgs(p, T);
   const int64_t P = (int64_t)NHG * pre_b + (int64_t)hg * n;
   // owners of the pair's first and last stages, and wf's slot (below); in
   // 32-bit arithmetic when T * (W + 1) < 2^32 (every product below is then
@@ -188,12 +202,8 @@ __device__ __forceinline__ void sk_merge_one(const MqParams& p, int b, int idx, 
   if (wf == wl) return;  // finished by its workgroup
   // Workgroups in (wf, wl] start inside the pair, so it is their first pair
   // (slot 0); wf holds it in slot 0 if its range starts at P, else in slot 1
-  // (its last pair).  With T >= W no range is empty; otherwise workgroups
-  // with empty ranges wrote nothing and are skipped.  (64-bit divisions are
-  // long instruction sequences: one per contributor made this pass
-  // instruction-bound when pairs are cut many times.)  Slot s of workgroup w
-  // for (hh, col) is at base + (2w + s) * wstride.
-  const bool may_be_empty = T < W;
+  // (its last pair).  No range is empty (sk_active_wgs).  Slot s of workgroup
+  // w for (hh, col) is at base + (2w + s) * wstride.
   const float* base = p.sk_part + (int64_t)(hh * p.sk_cols + col) * kSkSlotFloats;
   const int64_t wstride = (int64_t)HG * p.sk_cols * kSkSlotFloats;
   // Contributors in chunks of 16 (one DPP row): all of a chunk's loads
@@ -205,19 +215,11 @@ __device__ __forceinline__ void sk_merge_one(const MqParams& p, int b, int idx, 
   for (int w0 = wf; w0 <= wl; w0 += kChunk) {
     const int cnt = min(kChunk, wl - w0 + 1);
     float mi = -INFINITY, li = 0.f;
-    uint32_t skip = 0;  // bit j: contributor j has an empty range (only when T < W)
-    if (may_be_empty) {
-#pragma nounroll
-      for (int j = 0; j < cnt; ++j)
-        if (sk_range_start<uint32_t>(w0 + j, (uint32_t)T, W, a) ==  // T < W: T * C(W) < 2^32
-            sk_range_start<uint32_t>(w0 + j + 1, (uint32_t)T, W, a))
-          skip |= 1u << j;
-    }
     uint32_t a[kChunk];  // dims 2 lane, 2 lane + 1 of contributor j's acc / l (fp16)
 #pragma unroll
     for (int j = 0; j < kChunk; ++j) {
       a[j] = 0u;
-      if (j < cnt && !((skip >> j) & 1u)) {
+      if (j < cnt) {
         const int w = w0 + j;
         const float* ps = base + (int64_t)(2 * w + (w == wf ? slot_f : 0)) * wstride;
         a[j] = reinterpret_cast<const uint32_t*>(ps)[lane];
@@ -253,95 +255,138 @@ __device__ __forceinline__ void sk_merge_one(const MqParams& p, int b, int idx, 
   out[lane] = out_bits_rt(o0 * inv, f16) | (out_bits_rt(o1 * inv, f16) << 16);
 }
 
-// Decode (one query row per sequence) with G <= 4 query heads per kv head:
-// the merge of one (sequence, kv head) by one wave, 16 lanes per query head
-// (8 dims each), so a wave covers the kv head's G heads with the same two
-// memory round trips (the pair's prefix, then every contributor's partial) as
-// sk_merge_one takes for one head, and the launch has a quarter of the waves.
-// Every lane loads each contributor's (m, l) itself (the 16 lanes of a head
-// share the address), so no cross-lane exchange is needed; the contributors
-// are added in workgroup order.
-__device__ __forceinline__ void sk_merge_heads(const MqParams& p, int b, int kvh, int lane) {
-  const int G = p.G, HG = p.sk_heads, NHG = p.Hkv / HG;
-  const int sub = lane >> 4, d8 = lane & 15;  // query head kvh * G + sub, dims 8 d8 .. 8 d8 + 7
-  const int hg = kvh / HG, hh = kvh - hg * HG;
-  const int pre_b = p.sk_prefix[b];
-  const int n = p.sk_prefix[b + 1] - pre_b;
-  u32x4* out = reinterpret_cast<u32x4*>(p.out + ((int64_t)b * p.Hq + kvh * G + sub) * kHeadDim + 8 * d8);
-  if (n == 0) {
-    // Empty context (graph padding rows): the reference yields NaN here; write 0.
-    if (sub < G) *out = u32x4{0u, 0u, 0u, 0u};
-    return;
-  }
-  const int W = p.sk_wgs;
-  const int64_t T = (int64_t)NHG * p.sk_prefix[p.num_seqs];
-  const int64_t P = (int64_t)NHG * pre_b + (int64_t)hg * n;
-  const int a = sk_even_weight(p);
-  int wf, wl, slot_f;
-  if (sk_fits32(T, W, a)) sk_pair_owners<uint32_t>((uint32_t)P, (uint32_t)n, (uint32_t)T, (uint32_t)W, (uint32_t)a, wf, wl, slot_f);
-  else sk_pair_owners<uint64_t>((uint64_t)P, (uint64_t)n, (uint64_t)T, (uint64_t)W, (uint64_t)a, wf, wl, slot_f);
-  if (wf == wl) return;  // finished by its workgroup
-  // slot s of workgroup w for (hh, col) at base + (2w + s) * wstride (as in sk_merge_one)
-  const int col = min(sub, G - 1);
-  const float* base = p.sk_part + (int64_t)(hh * p.sk_cols + col) * kSkSlotFloats;
-  const int64_t wstride = (int64_t)HG * p.sk_cols * kSkSlotFloats;
-  const bool may_be_empty = T < W;  // then workgroups with empty ranges wrote nothing
-  float M = -INFINITY, L = 0.f, o[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) o[i] = 0.f;
-  for (int w0 = wf; w0 <= wl; w0 += 8) {
-    const int cnt = min(8, wl - w0 + 1);
-    uint32_t use = (1u << cnt) - 1u;  // bit j: contributor w0 + j wrote a partial
-    if (may_be_empty) {
-#pragma nounroll
-      for (int j = 0; j < cnt; ++j)
-        if (sk_range_start<uint32_t>(w0 + j, (uint32_t)T, W, a) ==  // T < W: T * C(W) < 2^32
-            sk_range_start<uint32_t>(w0 + j + 1, (uint32_t)T, W, a))
-          use &= ~(1u << j);
-    }
-    u32x4 h[8];
-    f32x2 ml[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {  // all of the chunk's loads before any is used: one round trip
-      // a contributor without a partial reads wl's instead (its weight is zero
-      // and the skipped slot may hold anything, NaN included)
-      const int w = ((use >> j) & 1u) ? w0 + j : wl;
-      const float* ps = base + (int64_t)(2 * w + (w == wf ? slot_f : 0)) * wstride;
-      h[j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(ps) + 8 * d8);
-      ml[j] = *reinterpret_cast<const f32x2*>(ps + kSkSlotMl);
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) mx = ((use >> j) & 1u) ? fmaxf(mx, ml[j].x) : mx;
-    const float Mn = fmaxf(M, mx);
+// State of a merge of up to four query columns of one kv head by one wave: 16
+// lanes per column, 8 dims each (m, l and the weighted sum of the partials'
+// normalised accumulators).
+struct SkMergeState {
+  float M = -INFINITY, L = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+  // Rescales to the maximum Mn (>= M) and returns it with -inf read as 0.
+  __device__ __forceinline__ float rescale(float Mn) {
     const float Ms = (Mn == -INFINITY) ? 0.f : Mn;
     const float sc = (M == -INFINITY) ? 0.f : fast_exp2(M - Ms);
     L *= sc;
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] *= sc;
     M = Mn;
+    return Ms;
+  }
+};
+
+// Adds the partials of workgroups w0, w0 + 1, .. min(w0 + 7, wl) in that
+// order.  All the loads are issued before any is used (one memory round
+// trip); workgroups past wl read wl's partial with weight zero.
+__device__ __forceinline__ void sk_merge_chunk(SkMergeState& st, const float* base, int64_t wstride, int w0, int wl,
+                                               int wf, int slot_f, int d8) {
+  u32x4 h[8];
+  f32x2 ml[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {  // weight of a normalised partial: w_j * l_j
-      const bool u = ((use >> j) & 1u) && ml[j].x != -INFINITY;
-      const float wk = u ? fast_exp2(ml[j].x - Ms) * ml[j].y : 0.f;
-      L += wk;
-      const uint32_t hw[4] = {h[j].x, h[j].y, h[j].z, h[j].w};
+  for (int j = 0; j < 8; ++j) {
+    const int w = min(w0 + j, wl);
+    const float* ps = base + (int64_t)(2 * w + (w == wf ? slot_f : 0)) * wstride;
+    h[j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(ps) + 8 * d8);
+    ml[j] = *reinterpret_cast<const f32x2*>(ps + kSkSlotMl);
+  }
+  float mx = st.M;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const f16x2 h2 = __builtin_bit_cast(f16x2, hw[e]);
-        o[2 * e] += wk * (float)h2.x;
-        o[2 * e + 1] += wk * (float)h2.y;
-      }
+  for (int j = 0; j < 8; ++j) mx = fmaxf(mx, ml[j].x);  // (repeats of wl change nothing)
+  const float Ms = st.rescale(mx);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {  // weight of a normalised partial: w_j * l_j
+    const bool u = w0 + j <= wl && ml[j].x != -INFINITY;
+    const float wk = u ? fast_exp2(ml[j].x - Ms) * ml[j].y : 0.f;
+    st.L += wk;
+    const uint32_t hw[4] = {h[j].x, h[j].y, h[j].z, h[j].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const f16x2 h2 = __builtin_bit_cast(f16x2, hw[e]);
+      st.o[2 * e] += wk * (float)h2.x;
+      st.o[2 * e + 1] += wk * (float)h2.y;
     }
   }
-  if (sub >= G) return;
-  const float inv = (L > 0.f) ? 1.0f / L : 0.f;
+}
+
+// Merge of up to four query columns (4 cg .. 4 cg + 3 of the kv head's
+// columns: column c is query row c / G, head c % G) of one (sequence, kv
+// head) by NW waves of a workgroup, 16 lanes per column: one wave covers four
+// columns with the two memory round trips (the pair's prefix, then every
+// contributor's partial) that sk_merge_one takes for one.  Every lane loads
+// each contributor's (m, l) itself (the 16 lanes of a column share the
+// address), so no cross-lane exchange is needed.
+// NW == 1: one wave takes the contributors eight at a time in workgroup
+// order.  NW > 1 (few pairs, so each is cut into up to W ranges): wave i takes
+// chunks i, i + NW, ..; the waves' states are combined in wave order through
+// `sm` (NW * 64 * 10 floats of LDS), so W / (8 NW) round trips in a row
+// instead of W / 8.  Every wave of the workgroup must call it.
+template <int NW>
+__device__ __forceinline__ void sk_merge_cols(const MqParams& p, int b, int kvh, int cg, int wave, int lane, float* sm) {
+  const int G = p.G, HG = p.sk_heads, NHG = p.Hkv / HG;
+  const int sub = lane >> 4, d8 = lane & 15;  // column 4 cg + sub, dims 8 d8 .. 8 d8 + 7
+  const int hg = kvh / HG, hh = kvh - hg * HG;
+  int64_t q0 = b;
+  int lq = 1;
+  if (p.cu_q != nullptr) {  // varlen: short-query sequences only
+    q0 = p.cu_q[b];
+    lq = p.cu_q[b + 1] - (int)q0;
+    if (lq <= 0 || lq > p.mq_max_q) return;
+  }
+  const int pre_b = p.sk_prefix[b];
+  const int n = p.sk_prefix[b + 1] - pre_b;
+  const int c0 = 4 * cg + sub, qr = c0 / G;
+  const bool valid = qr < lq && q0 + qr < p.q_rows;
+  u32x4* out = reinterpret_cast<u32x4*>(p.out + ((q0 + qr) * p.Hq + kvh * G + (c0 - qr * G)) * kHeadDim + 8 * d8);
+  if (n == 0) {
+    // Empty context (graph padding rows): the reference yields NaN here; write 0.
+    if (valid && wave == 0) *out = u32x4{0u, 0u, 0u, 0u};
+    return;
+  }
+  const int64_t T = (int64_t)NHG * p.sk_prefix[p.num_seqs];
+  const int W = sk_active_wgs(p, T);
+  const int64_t P = (int64_t)NHG * pre_b + (int64_t)hg * n;
+  const int a = sk_even_weight(p);
+  int wf, wl, slot_f;
+  if (sk_fits32(T, W, a)) sk_pair_owners<uint32_t>((uint32_t)P, (uint32_t)n, (uint32_t)T, (uint32_t)W, (uint32_t)a, wf, wl, slot_f);
+  else sk_pair_owners<uint64_t>((uint64_t)P, (uint64_t)n, (uint64_t)T, (uint64_t)W, (uint64_t)a, wf, wl, slot_f);
+  if (wf == wl) return;  // finished by its workgroup
+  // slot s of workgroup w for (hh, col) at base + (2w + s) * wstride (as in
+  // sk_merge_one); a lane without a column reads the slot's last one
+  const int col = min(c0, p.sk_cols - 1);
+  const float* base = p.sk_part + (int64_t)(hh * p.sk_cols + col) * kSkSlotFloats;
+  const int64_t wstride = (int64_t)HG * p.sk_cols * kSkSlotFloats;
+  SkMergeState st;
+  if (NW == 1 || wl - wf < 8) {
+    if (wave > 0) return;
+    for (int w0 = wf; w0 <= wl; w0 += 8) sk_merge_chunk(st, base, wstride, w0, wl, wf, slot_f, d8);
+  } else {
+    for (int w0 = wf + 8 * wave; w0 <= wl; w0 += 8 * NW) sk_merge_chunk(st, base, wstride, w0, wl, wf, slot_f, d8);
+    if (wave > 0) {
+      float* mine = sm + wave * 640 + lane;  // [wave][value][lane]
+      mine[0] = st.M;
+      mine[64] = st.L;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mine[64 * (2 + i)] = st.o[i];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int k = 1; k < NW; ++k) {  // a wave without a chunk left m = -inf
+      const float* other = sm + k * 640 + lane;
+      const float mk = other[0];
+      const float Ms = st.rescale(fmaxf(st.M, mk));
+      const float wk = (mk == -INFINITY) ? 0.f : fast_exp2(mk - Ms);
+      st.L += wk * other[64];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) st.o[i] += wk * other[64 * (2 + i)];
+    }
+  }
+  if (!valid) return;
+  const float inv = (st.L > 0.f) ? 1.0f / st.L : 0.f;
   const bool f16 = p.out_f16 != 0;
   u32x4 v;
-  v.x = out_bits_rt(o[0] * inv, f16) | (out_bits_rt(o[1] * inv, f16) << 16);
-  v.y = out_bits_rt(o[2] * inv, f16) | (out_bits_rt(o[3] * inv, f16) << 16);
-  v.z = out_bits_rt(o[4] * inv, f16) | (out_bits_rt(o[5] * inv, f16) << 16);
-  v.w = out_bits_rt(o[6] * inv, f16) | (out_bits_rt(o[7] * inv, f16) << 16);
+  v.x = out_bits_rt(st.o[0] * inv, f16) | (out_bits_rt(st.o[1] * inv, f16) << 16);
+  v.y = out_bits_rt(st.o[2] * inv, f16) | (out_bits_rt(st.o[3] * inv, f16) << 16);
+  v.z = out_bits_rt(st.o[4] * inv, f16) | (out_bits_rt(st.o[5] * inv, f16) << 16);
+  v.w = out_bits_rt(st.o[6] * inv, f16) | (out_bits_rt(st.o[7] * inv, f16) << 16);
   *out = v;
 }
 

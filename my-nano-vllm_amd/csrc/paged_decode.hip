@@ -686,7 +686,6 @@ __global__ __launch_bounds__(64 * HG) void decode_sk_kernel(MqParams p, PrefillP
   const int G = p.G;
   const int NHG = p.Hkv / HG;
   const int B = p.num_seqs;
-  const int W = p.sk_wgs;
   const int w = blockIdx.x;
   constexpr int kThreads = 64 * HG;
   const int cap = sk_capacity(p);
@@ -716,6 +715,8 @@ __global__ __launch_bounds__(64 * HG) void decode_sk_kernel(MqParams p, PrefillP
   if (w == 0)
     for (int b = tid; b <= B; b += kThreads) p.sk_prefix[b] = pre[b];
   // this workgroup's share of the stages (sk_range_start)
+  const int W = sk_active_wgs(p, T);
+  if (w >= W) return;
   int64_t start, end;
   {
     const int a = sk_even_weight(p);
@@ -1023,7 +1024,19 @@ __global__ __launch_bounds__(256) void decode_sk_merge_heads_kernel(MqParams p) 
   const int gw = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
   if (gw >= p.num_seqs * p.Hkv) return;
   const int b = gw / p.Hkv;
-  sk_merge_heads(p, b, gw - b * p.Hkv, threadIdx.x & 63);
+  sk_merge_cols<1>(p, b, gw - b * p.Hkv, 0, 0, threadIdx.x & 63, nullptr);
+}
+
+// Few pairs: a workgroup of kSkWideWaves waves per (sequence, kv head, four
+// query columns), the contributors dealt over the waves.
+constexpr int kSkWideWaves = 8;
+constexpr int64_t kSkWideMaxWgs = 1024;
+__global__ __launch_bounds__(64 * kSkWideWaves) void decode_sk_merge_wide_kernel(MqParams p, int groups) {
+  __shared__ float sm[kSkWideWaves * 640];
+  // 32-bit index: the launch takes this kernel for at most kSkWideMaxWgs workgroups
+  const int pair = (int)blockIdx.x / groups, cg = (int)blockIdx.x - pair * groups;
+  const int b = pair / p.Hkv;
+  sk_merge_cols<kSkWideWaves>(p, b, pair - b * p.Hkv, cg, wave_uniform(threadIdx.x >> 6), threadIdx.x & 63, sm);
 }
 
 namespace {
@@ -1101,7 +1114,17 @@ hipError_t launch_decode_sk(const MqParams& p, int ncb, bool merge, const Prefil
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (!merge) return hipSuccess;  // the caller's next launch merges
-  if (!varlen && p.G <= 4)
+  // Few pairs (at most kSkWideMaxWgs workgroups, four a CU): a pair may be cut
+  // into as many ranges as there are workgroups, and one wave adding them in
+  // turn is a chain of up to W / 8 memory round trips (one 131,072-token
+  // sequence on 32 / 8 heads: 80.8 us per call with one wave a pair, 53.1 with
+  // eight; 8 sequences of 256-4,096: 24.2 and 18.4).
+  const int groups = (p.G * p.mq_max_q + 3) / 4;  // of four query columns
+  const int64_t wide_wgs = (int64_t)p.num_seqs * p.Hkv * groups;
+  if (wide_wgs <= kSkWideMaxWgs)
+    hipLaunchKernelGGL(decode_sk_merge_wide_kernel, dim3((unsigned)wide_wgs), dim3(64 * kSkWideWaves), 0, stream, p,
+                       groups);
+  else if (!varlen && p.G <= 4)
     hipLaunchKernelGGL(decode_sk_merge_heads_kernel, dim3((unsigned)(((int64_t)p.num_seqs * p.Hkv + 3) / 4)),
                        dim3(256), 0, stream, p);
   else

@@ -159,3 +159,33 @@ def test_balanced_decode_garbage_and_reused_workspace():
         _native.check(st, "decode")
         torch.cuda.synchronize()
         assert_close(out, want, f"garbage_ws call {call}")
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (64, 8), (8, 4), (24, 8)])
+@pytest.mark.parametrize("ctx", [[1], [16], [17], [33], [49], [777], [4079], [4096], [8191], [16400], [40000],
+                                 [5, 0, 700], [1, 9000, 64], [300] * 5], ids=str)
+def test_balanced_decode_few_pairs(hq, hkv, ctx):
+    """Few pairs: from one stage on one workgroup, over calls that use half of
+    the grid (two to four stages each), to pairs cut into every range, whose
+    partials several waves combine; after a call that left the workspace's
+    partials full of another call's values."""
+    seqs = [W.SeqSpec(lq=1, cached=max(c, 1) - 1) for c in ctx]
+    wl = W.make_workload(f"few_{hq}_{hkv}_{ctx}", hq, hkv, seqs, seed=sum(ctx) + hq)
+    announce(f"balanced decode: few pairs {hq}/{hkv} ctx={ctx}")
+    cpu_c, gpu_c = build_pair(wl, gen_device="cuda")
+    q = wl.make_q("cpu")
+    ctx_t = torch.tensor(ctx, dtype=torch.int32)
+    lib = _native.load()
+    bt = torch.from_numpy(wl.block_tables).cuda()
+    need = lib.nvamd_decode_workspace_bytes(len(ctx), hq, hkv, bt.shape[1], 256, 0)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")  # NaN wherever nothing was written
+    out, qg, ctx_g = torch.empty(q.shape, dtype=q.dtype, device="cuda"), q.cuda(), ctx_t.cuda()
+    st = lib.nvamd_fp8_decode_attention(out.data_ptr(), qg.data_ptr(), gpu_c[0].data_ptr(), gpu_c[1].data_ptr(),
+                                        bt.data_ptr(), ctx_g.data_ptr(), len(ctx), hq, hkv, 128, wl.num_blocks, 256,
+                                        bt.shape[1], SCALE, 0, ws.data_ptr(), need, 0,
+                                        torch.cuda.current_stream().cuda_stream)
+    _native.check(st, "decode")
+    torch.cuda.synchronize()
+    keep = ctx_t > 0
+    assert bool((out.cpu()[~keep] == 0).all()), "empty-context rows must be 0"
+    assert_close(out, _oracle(wl, cpu_c, q, ctx_t), wl.name, mask_rows=keep)
