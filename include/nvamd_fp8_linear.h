@@ -74,6 +74,23 @@ int32_t nvamd_fp8_block_gemm(const void* xq, const void* x_scale, const void* we
  * current device (0: none). */
 int64_t nvamd_fp8_block_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
+/*
+ * The whole linear layer: nvamd_fp8_act_quant, then nvamd_fp8_block_gemm
+ * (arguments as theirs; out has x's type).  A call of a few tokens is one
+ * kernel that quantises its activations itself.
+ *
+ * workspace (16-byte aligned, contents ignored):
+ * nvamd_fp8_block_linear_workspace_bytes(M, N, K) bytes; NULL with
+ * workspace_bytes 0 when that is 0.
+ */
+int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype, const void* weight,
+                               int64_t weight_stride0, const void* weight_scale, void* out, int64_t out_stride0,
+                               int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Workspace bytes nvamd_fp8_block_linear uses for an M x N x K product on the
+ * current device (0: none). */
+int64_t nvamd_fp8_block_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
 #ifdef __cplusplus
 }
 #endif

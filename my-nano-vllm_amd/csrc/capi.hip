@@ -337,10 +337,13 @@ int64_t nvamd_fp8_block_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return nvamd::fp8_skinny_workspace_bytes(M, N, (int)(K / 128), device_cu_count(), device_lds_limit());
 }
 
-int32_t nvamd_fp8_block_gemm(const void* xq, const void* x_scale, const void* weight, int64_t weight_stride0,
-                             const void* weight_scale, void* out, int64_t out_stride0, int32_t out_dtype, int64_t M,
-                             int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
-  static const char* fn = "fp8_block_gemm";
+namespace {
+
+// Checks of a product's sizes and operands shared by the GEMM and the whole
+// linear (x is xq or the raw activations).
+int32_t check_linear(const char* fn, const void* x, const void* weight, int64_t weight_stride0, const void* weight_scale,
+                     const void* out, int64_t out_stride0, int32_t out_dtype, int64_t M, int64_t N, int64_t K,
+                     const void* workspace, int64_t workspace_bytes) {
   if (M < 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || weight_stride0 < K || out_stride0 < N ||
       N > 0x7fffffffll || K > 0x7fffffffll)
     return fail(NVAMD_ERR_INVALID_ARGUMENT, "%s: bad sizes (M=%lld N=%lld K=%lld; N, K multiples of 128)", fn,
@@ -353,22 +356,21 @@ int32_t nvamd_fp8_block_gemm(const void* xq, const void* x_scale, const void* we
                 (long long)workspace_bytes);
   if ((uintptr_t)workspace % 16 != 0)
     return fail(NVAMD_ERR_UNSUPPORTED, "%s: workspace must be 16-byte aligned", fn);
-  if (!xq || !x_scale || !weight || !weight_scale || !out) return fail(NVAMD_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
-  if ((uintptr_t)xq % 16 != 0 || (uintptr_t)x_scale % 16 != 0 || (uintptr_t)weight % 16 != 0 ||
-      weight_stride0 % 16 != 0 || (uintptr_t)weight_scale % 16 != 0 || (uintptr_t)out % 8 != 0 || out_stride0 % 4 != 0)
+  if (!x || !weight || !weight_scale || !out) return fail(NVAMD_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
+  if ((uintptr_t)x % 16 != 0 || (uintptr_t)weight % 16 != 0 || weight_stride0 % 16 != 0 ||
+      (uintptr_t)weight_scale % 16 != 0 || (uintptr_t)out % 8 != 0 || out_stride0 % 4 != 0)
     return fail(NVAMD_ERR_UNSUPPORTED,
                 "%s: operands must be 16-byte aligned (out 8), weight row stride a multiple of 16 bytes, out row stride "
                 "a multiple of 4 elements",
                 fn);
   if (weight_stride0 * 256 > 0xffffffffll || M * K > (1ll << 46))
     return fail(NVAMD_ERR_UNSUPPORTED, "%s: weight row stride or activation size beyond 32-bit tile offsets", fn);
-  const int64_t lds_limit = device_lds_limit();
-  const int Kc = (int)(K / 128);
-  const nvamd::SkinnyPlan plan = nvamd::fp8_skinny_plan(M, N, Kc, device_cu_count(), workspace_bytes, lds_limit);
-  const int config = plan.cw > 0 ? 0 : nvamd::fp8_gemm_pick_config(M, N, Kc, device_cu_count(), lds_limit);
-  if (config < 0)
-    return fail(NVAMD_ERR_UNSUPPORTED, "%s: K=%lld needs more LDS for the tile scales than the device has", fn,
-                (long long)K);
+  return NVAMD_OK;
+}
+
+nvamd::Fp8GemmParams gemm_params(const void* xq, const void* x_scale, const void* weight, int64_t weight_stride0,
+                                 const void* weight_scale, void* out, int64_t out_stride0, int64_t M, int64_t N,
+                                 int64_t K) {
   nvamd::Fp8GemmParams p{};
   p.xq = static_cast<const uint8_t*>(xq);
   p.x_scale = static_cast<const uint16_t*>(x_scale);
@@ -380,12 +382,78 @@ int32_t nvamd_fp8_block_gemm(const void* xq, const void* x_scale, const void* we
   p.M = M;
   p.N = (int)N;
   p.K = (int)K;
-  p.Kc = Kc;
+  p.Kc = (int)(K / 128);
+  return p;
+}
+
+// The GEMM on quantised activations: the kernel its sizes call for.
+int32_t run_block_gemm(const char* fn, const nvamd::Fp8GemmParams& p, bool f16_out, void* workspace,
+                       int64_t workspace_bytes, hipStream_t stream) {
+  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(p.M, p.N, p.Kc, device_cu_count(), false);
+  if (thin.mf > 0)
+    return launch_status(nvamd::launch_fp8_thin_linear(p, thin, nullptr, 0, false, f16_out, stream), fn);
+  const int64_t lds_limit = device_lds_limit();
+  const nvamd::SkinnyPlan plan = nvamd::fp8_skinny_plan(p.M, p.N, p.Kc, device_cu_count(), workspace_bytes, lds_limit);
   if (plan.cw > 0)
-    return launch_status(nvamd::launch_fp8_skinny_gemm(p, plan, out_dtype == NVAMD_DTYPE_F16,
-                                                       static_cast<float*>(workspace), (hipStream_t)stream),
-                         fn);
-  return launch_status(nvamd::launch_fp8_block_gemm(p, config, out_dtype == NVAMD_DTYPE_F16, (hipStream_t)stream), fn);
+    return launch_status(nvamd::launch_fp8_skinny_gemm(p, plan, f16_out, static_cast<float*>(workspace), stream), fn);
+  const int config = nvamd::fp8_gemm_pick_config(p.M, p.N, p.Kc, device_cu_count(), lds_limit);
+  if (config < 0)
+    return fail(NVAMD_ERR_UNSUPPORTED, "%s: K=%lld needs more LDS for the tile scales than the device has", fn,
+                (long long)p.K);
+  return launch_status(nvamd::launch_fp8_block_gemm(p, config, f16_out, stream), fn);
+}
+
+// nvamd_fp8_block_linear's scratch: the quantised activations and their
+// scales, then (256-byte aligned) the GEMM's workspace.
+int64_t act_bytes(int64_t M, int64_t K) { return align_up(align_up(M * K) + M * (K / 128) * 2); }
+
+}  // namespace
+
+int32_t nvamd_fp8_block_gemm(const void* xq, const void* x_scale, const void* weight, int64_t weight_stride0,
+                             const void* weight_scale, void* out, int64_t out_stride0, int32_t out_dtype, int64_t M,
+                             int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
+  static const char* fn = "fp8_block_gemm";
+  if (int32_t e = check_linear(fn, xq, weight, weight_stride0, weight_scale, out, out_stride0, out_dtype, M, N, K,
+                               workspace, workspace_bytes))
+    return e;
+  if (M == 0) return ok();
+  if (!x_scale) return fail(NVAMD_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
+  if ((uintptr_t)x_scale % 16 != 0) return fail(NVAMD_ERR_UNSUPPORTED, "%s: operands must be 16-byte aligned", fn);
+  return run_block_gemm(fn, gemm_params(xq, x_scale, weight, weight_stride0, weight_scale, out, out_stride0, M, N, K),
+                        out_dtype == NVAMD_DTYPE_F16, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int64_t nvamd_fp8_block_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > 0x7fffffffll || K > 0x7fffffffll) return 0;
+  if (nvamd::fp8_thin_plan(M, N, (int)(K / 128), device_cu_count(), true).xi > 0) return 0;
+  return act_bytes(M, K) + nvamd_fp8_block_gemm_workspace_bytes(M, N, K);
+}
+
+int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype, const void* weight,
+                               int64_t weight_stride0, const void* weight_scale, void* out, int64_t out_stride0,
+                               int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
+  static const char* fn = "fp8_block_linear";
+  if (int32_t e = check_linear(fn, x, weight, weight_stride0, weight_scale, out, out_stride0, x_dtype, M, N, K,
+                               workspace, workspace_bytes))
+    return e;
+  if (x_stride0 < K) return fail(NVAMD_ERR_INVALID_ARGUMENT, "%s: x row stride is shorter than a row", fn);
+  if (x_stride0 % 8 != 0) return fail(NVAMD_ERR_UNSUPPORTED, "%s: x row stride must be a multiple of 8 elements", fn);
+  if (M == 0) return ok();
+  const bool f16 = x_dtype == NVAMD_DTYPE_F16;
+  nvamd::Fp8GemmParams p =
+      gemm_params(nullptr, nullptr, weight, weight_stride0, weight_scale, out, out_stride0, M, N, K);
+  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(M, N, p.Kc, device_cu_count(), true);
+  if (thin.xi > 0)
+    return launch_status(nvamd::launch_fp8_thin_linear(p, thin, x, x_stride0, f16, f16, (hipStream_t)stream), fn);
+  const int64_t act = act_bytes(M, K);
+  if (workspace_bytes < act)
+    return fail(NVAMD_ERR_WORKSPACE, "%s: workspace of %lld bytes needed", fn, (long long)act);
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  p.xq = ws;
+  p.x_scale = reinterpret_cast<const uint16_t*>(ws + align_up(M * K));
+  if (int32_t e = nvamd_fp8_act_quant(x, x_stride0, x_dtype, ws, ws + align_up(M * K), M, K, stream)) return e;
+  const int64_t left = workspace_bytes - act;
+  return run_block_gemm(fn, p, f16, left > 0 ? ws + act : nullptr, left, (hipStream_t)stream);
 }
 
 int32_t nvamd_build_attention_metadata(const int32_t* packed, int64_t packed_ints, int32_t num_seqs, int32_t num_plain,

@@ -40,6 +40,7 @@
 #include <cmath>
 
 #include "fp8_common.h"
+#include "fp8_quant.h"
 #include "kernels.h"
 #include "lds_dma.h"
 
@@ -49,17 +50,9 @@ namespace {
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kFp8Block = 128;  // the reference's BLOCK_SIZE (fp8_linear.py:8)
-
 // ---------------------------------------------------------------------------
 // Dynamic activation quantisation
 // ---------------------------------------------------------------------------
-template <bool F16_IN>
-__device__ __forceinline__ float in_to_f32(uint32_t bits16) {
-  if constexpr (F16_IN) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
-  return bf16_bits_to_f32(bits16);
-}
-
 // Grid (M, ceil(Kc / 16)): workgroup (m, y) quantises groups 16 y .. 16 y + 15
 // of token m, one 16-lane group each, so no lane divides.
 template <bool F16_IN>
@@ -71,25 +64,10 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
   const int j = (int)(threadIdx.x & 15);
   if (g >= Kc) return;  // whole 16-lane groups
   const u32x4 w = *reinterpret_cast<const u32x4*>(x + m * x_stride + (int64_t)g * kFp8Block + 8 * j);
-  const uint32_t d[4] = {w.x, w.y, w.z, w.w};
-  float v[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    v[2 * i] = in_to_f32<F16_IN>(d[i] & 0xFFFFu);
-    v[2 * i + 1] = in_to_f32<F16_IN>(d[i] >> 16);
-  }
-  float amax = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) amax = fmaxf(amax, __builtin_fabsf(v[i]));
-  amax = row16_max(amax);  // the group's 16 lanes are one DPP row
-  float scale = amax / 448.0f;  // correctly rounded fp32 division
-  scale = scale > 0.f ? scale : 1.0f;
-  float y[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) y[i] = v[i] / scale;  // clamp and RNE in f32x4_to_fp8x4
+  float scale;
   *reinterpret_cast<u32x2*>(xq + m * ((int64_t)Kc * kFp8Block) + (int64_t)g * kFp8Block + 8 * j) =
-      u32x2{f32x4_to_fp8x4(y[0], y[1], y[2], y[3]), f32x4_to_fp8x4(y[4], y[5], y[6], y[7])};
-  if (j == 0) x_scale[m * Kc + g] = (uint16_t)(pack_bf16x2(scale, 0.f) & 0xFFFFu);
+      quant_group8<F16_IN>(w, scale);
+  if (j == 0) x_scale[m * Kc + g] = (uint16_t)scale_bf16_bits(scale);
 }
 
 // ---------------------------------------------------------------------------

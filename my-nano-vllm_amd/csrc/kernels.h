@@ -170,6 +170,18 @@ int64_t fp8_skinny_workspace_bytes(int64_t M, int64_t N, int Kc, int cus, int64_
 hipError_t launch_fp8_skinny_gemm(const Fp8GemmParams& p, const SkinnyPlan& plan, bool f16_out, float* part,
                                   hipStream_t stream);
 
+// Linear for at most kThinMaxM tokens in one launch (fp8_thin_linear.hip): nw
+// waves per workgroup, mf 16-token fragments; xi > 0: the kernel quantises x
+// itself (xi passes of four groups per wave and chunk), else it reads the
+// quantised activations.  mf == 0: no plan.
+constexpr int64_t kThinMaxM = 32;
+struct ThinPlan {
+  int nw = 0, mf = 0, xi = 0;
+};
+ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, bool raw_x);
+hipError_t launch_fp8_thin_linear(const Fp8GemmParams& p, const ThinPlan& plan, const void* x, int64_t x_stride,
+                                  bool f16_in, bool f16_out, hipStream_t stream);
+
 hipError_t launch_kv_store(const void* key, int64_t key_stride, const void* value,
                            int64_t value_stride, void* k_cache, void* v_cache,
                            const int32_t* slot_mapping, int64_t num_tokens, int row_elems,

@@ -247,18 +247,13 @@ at::Tensor fp8_block_linear(const at::Tensor& x_in, const at::Tensor& w_in, cons
   const at::Tensor wsc = (ws_in.scalar_type() == at::kBFloat16 ? ws_in : ws_in.to(at::kBFloat16)).contiguous();
   const at::OptionalDeviceGuard guard(x.device());
   const hipStream_t stream = stream_of(x);
-  // the quantised activations [M, K] and their bf16 scales [M, K/128], one allocation
-  const int64_t xq_bytes = (M * K + 255) / 256 * 256;
-  const c10::DataPtr act = workspace(xq_bytes + M * (K / 128) * 2);
-  void* xq = act.get();
-  void* x_scale = static_cast<char*>(act.get()) + xq_bytes;
-  check_status(nvamd_fp8_act_quant(x.data_ptr(), x.stride(0), dt, xq, x_scale, M, K, stream), "fp8_act_quant");
   at::Tensor out = at::empty({M, N}, x.options());
-  const int64_t ws_n = nvamd_fp8_block_gemm_workspace_bytes(M, N, K);
+  const int64_t ws_n = nvamd_fp8_block_linear_workspace_bytes(M, N, K);
   const c10::DataPtr ws = workspace(ws_n);
-  check_status(nvamd_fp8_block_gemm(xq, x_scale, w.data_ptr(), w.stride(0), wsc.data_ptr(), out.data_ptr(),
-                                    out.stride(0), dt, M, N, K, ws.get(), ws.get() != nullptr ? ws_n : 0, stream),
-               "fp8_block_gemm");
+  check_status(nvamd_fp8_block_linear(x.data_ptr(), x.stride(0), dt, w.data_ptr(), w.stride(0), wsc.data_ptr(),
+                                      out.data_ptr(), out.stride(0), M, N, K, ws.get(),
+                                      ws.get() != nullptr ? ws_n : 0, stream),
+               "fp8_block_linear");
   return out;
 }
 

@@ -55,6 +55,9 @@ SIGNATURES = {
     "nvamd_fp8_block_gemm": (_i32, [_c_void_p, _c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p, _i64, _i32,
                                     _i64, _i64, _i64, _c_void_p, _i64, _c_void_p]),
     "nvamd_fp8_block_gemm_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "nvamd_fp8_block_linear": (_i32, [_c_void_p, _i64, _i32, _c_void_p, _i64, _c_void_p, _c_void_p, _i64,
+                                      _i64, _i64, _i64, _c_void_p, _i64, _c_void_p]),
+    "nvamd_fp8_block_linear_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "nvamd_prefill_workspace_bytes": (_i64, [_i64, _i32, _i32, _i32, _i64, _i32, _i32, _i32]),
     "nvamd_fp8_prefill_attention": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                            _c_void_p, _c_void_p, _i64, _i32, _i32, _i32, _i32,

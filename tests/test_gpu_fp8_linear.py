@@ -303,3 +303,63 @@ def test_skinny_gemm_matches_oracle(M, N, K, out_dtype):
     ulp = 2.0 ** -7 if out_dtype == torch.bfloat16 else 2.0 ** -10
     bad = (got - acc).abs() > ulp * acc.abs() + ABS_TOL * absum
     assert not bad.any(), f"{int(bad.sum())} outputs off, first at {bad.nonzero()[0].tolist()}"
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(128, 128), (256, 1024), (384, 1152), (1024, 3072), (4224, 640), (4352, 2176),
+                                 (512, 12288), (4224, 5248)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_tokens(M, N, K, dtype):
+    """Calls of at most 32 tokens: one K block to several chunks of eight per
+    wave with a short last one, one to eight waves, one workgroup a CU or more,
+    activations quantised in the kernel (up to 2 or 4 tokens) and read
+    quantised, strided activation rows.  Random codes against the oracle; the
+    same call on activations quantised beforehand adds the same products in
+    the same order, so it gives the same bits."""
+    g = torch.Generator().manual_seed(M + 3 * N + K)
+    wide = (torch.randn(M, K + 72, generator=g) * 3).to(dtype)
+    wide[0, :128] = 0.0                        # a group of zeros, with both signs
+    wide[0, 1:128:2] = -0.0
+    w, w_scale = _codes(g, (N, K)), (torch.rand(N // 128, K // 128, generator=g) * 2e-3).to(torch.bfloat16)
+    announce(f"fp8 linear: few tokens M={M} N={N} K={K} {dtype}")
+    x = wide.cuda()[:, :K]
+    got = fp8_block_linear(x, w.cuda().view(torch.float8_e4m3fn), w_scale.cuda())
+    torch.cuda.synchronize()
+    xq, xs, _ = ol.act_quant(wide[:, :K].contiguous())
+    xq, xs = torch.from_numpy(xq), torch.from_numpy(xs.view(np.int16)).view(torch.bfloat16)
+    pre = _gemm_gpu(xq, xs, w, w_scale, dtype)
+    assert torch.equal(got.cpu().view(torch.int16), pre.view(torch.int16)), "in-kernel quantisation differs"
+    _, acc = ol.block_gemm(xq.numpy(), _bits(xs), w.numpy(), _bits(w_scale), "bf16" if dtype == torch.bfloat16 else "fp16")
+    _, absum = _f64(xq, xs, w, w_scale)
+    acc = torch.from_numpy(acc).double()
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    bad = (got.cpu().double() - acc).abs() > ulp * acc.abs() + ABS_TOL * absum
+    assert not bad.any(), f"{int(bad.sum())} outputs off, first at {bad.nonzero()[0].tolist()}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_act_quant_edge_groups(dtype):
+    """Groups at the ends of the range the reciprocal form of the division
+    covers: signed zeros, subnormal values, the largest and smallest amax of
+    the type, a single value beside its smallest ones."""
+    announce(f"fp8 linear: activation quant, edge groups {dtype}")
+    info = torch.finfo(dtype)
+    tiny = info.smallest_normal * info.eps                   # the smallest subnormal
+    rows = [torch.zeros(128), -torch.zeros(128), torch.full((128,), tiny), torch.linspace(-1, 1, 128) * info.max,
+            torch.linspace(-1, 1, 128) * info.smallest_normal, torch.arange(128.0) * tiny]
+    if dtype == torch.bfloat16:                              # scales on both sides of 2^-100 and 2^100
+        rows += [torch.linspace(-1, 1, 128) * 448.0 * 2.0 ** e for e in (-101, -100, -99, 99, 100, 101)]
+    x = torch.stack([r.to(dtype) for r in rows] * 2)
+    x[len(rows):, 5] = info.max                              # ... beside the largest value
+    x = x.reshape(len(rows) * 2 // 2, 256)
+    xq_ref, xs_ref, _ = ol.act_quant(x)
+    lib = _native.load()
+    xd = x.cuda()
+    M, K = x.shape
+    xq = torch.empty(M, K, dtype=torch.uint8, device="cuda")
+    xs = torch.empty(M, K // 128, dtype=torch.bfloat16, device="cuda")
+    _native.check(lib.nvamd_fp8_act_quant(xd.data_ptr(), K, 0 if dtype == torch.bfloat16 else 1, xq.data_ptr(),
+                                          xs.data_ptr(), M, K, torch.cuda.current_stream().cuda_stream), "act_quant")
+    torch.cuda.synchronize()
+    assert np.array_equal(xq.cpu().numpy(), xq_ref)
+    assert np.array_equal(_bits(xs), xs_ref)
