@@ -287,6 +287,284 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
   }
 }
 
+// Tile (x, y) of workgroup `id` of a gx x gy grid launched as one row.
+// Workgroups go to the eight XCDs in turn, so XCD c (id % 8) takes a contiguous
+// run of the tiles, in an order whose neighbours share operands in its L2:
+// groups of G rows, inside a group column by column (its 32 resident
+// workgroups then cover 32 / G columns x G rows).
+template <int G>
+__device__ __forceinline__ void tile_of_block(int id, int gx, int gy, int& x, int& y) {
+  const int total = gx * gy, c = id & 7;
+  const int t = c * (total >> 3) + min(c, total & 7) + (id >> 3);
+  const int group = t / (G * gx), in = t - group * (G * gx);
+  const int rows = min(G, gy - group * G);
+  x = in / rows;
+  y = group * G + in - x * rows;
+}
+
+// ---------------------------------------------------------------------------
+// Large tiles: two wave groups that take turns on the matrix cores
+// ---------------------------------------------------------------------------
+// Eight waves, two per SIMD; waves 0-3 (one on each SIMD) and waves 4-7 work
+// half a K block apart.  In a phase one group runs its MFMAs from registers,
+// the other reads its next K block's fragments from LDS; one barrier ends the
+// phase and the groups swap.  With all eight waves in step (the tile kernel
+// above at this size) every K block began with both waves of a SIMD reading
+// fragments and issuing loads, matrix cores idle: 4,400 cycles per K block of
+// the 256 x 256 tile, of which the MFMAs are 2,048.
+//  - Within a phase an MFMA is followed by the four FMAs of the product three
+//    MFMAs back: 34 cycles per MFMA of one wave (register-only loop; 43 with a
+//    distance of two, 71 with one), so the block scales cost no MFMA slots.
+//  - Direct-to-LDS loads stall the wave that issues them (about 17 cycles each
+//    with the CU's address path free, 64 per K block): they are spread between
+//    the MFMAs of a phase.
+//  - What the tile reaches is set by the power limit: 4,400 -> 3,300 cycles
+//    per K block came with a clock of 1.36 instead of 1.68 GHz.
+template <int WN, int WM, int TN, int TM, int S, bool F16_OUT>
+__global__ __launch_bounds__(512) void swap_gemm_kernel(Fp8GemmParams p) {
+  using T = GemmTile<WN, WM, TN, TM, S>;
+  static_assert(WN * WM == 8 && WN <= 4, "two waves per SIMD; a group's waves share their half of the tokens");
+  static_assert(!T::kStraddle && (S == 2 || S == 3), "one weight block per wave; the load schedules below");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const uint32_t lds0 = wave_uniform((int)lds_addr(smem));
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6);
+  const int wn = wave % WN, wm = wave / WN;
+  const bool first = wave < 4;
+  int tx, ty;
+  tile_of_block<4>((int)blockIdx.x, p.N / T::BN, (int)((p.M + T::BM - 1) / T::BM), tx, ty);
+  const int n0 = tx * T::BN;
+  const int64_t m0 = (int64_t)ty * T::BM;
+  const int Kc = p.Kc;
+  const int rows_x = (int)min((int64_t)T::BM, p.M - m0);  // valid token rows of the tile
+
+  // descriptors as in the tile kernel
+  const u32x4 rw = rsrc_words(p.w + (int64_t)n0 * p.w_stride, (uint32_t)((int64_t)T::BN * p.w_stride));
+  const u32x4 rx = rsrc_words(p.xq + m0 * ((int64_t)Kc * kFp8Block), (uint32_t)((int64_t)rows_x * Kc * kFp8Block));
+  const int64_t sx_bytes = ((int64_t)rows_x * Kc * 2 + 3) & ~(int64_t)3;
+  const u32x4 rsx = rsrc_words(p.x_scale + m0 * Kc, (uint32_t)sx_bytes);
+  const int64_t sw_first = (int64_t)(n0 / kFp8Block) * Kc;
+  const int sw_shift = (int)(sw_first & 7);
+  const int64_t sw_elems = (int64_t)T::kWBlocks * Kc + sw_shift;
+  const u32x4 rsw = rsrc_words(p.w_scale + (sw_first - sw_shift), (uint32_t)((sw_elems * 2 + 3) & ~3ll));
+
+  // One load brings 8 rows x 128 B: lane l -> row + l / 8, granule position l % 8.
+  // A wave's loads are 32 rows apart (so the swizzle (r >> 1) & 7 is that of
+  // its first row).
+  const int fr = lane >> 3, fp = lane & 7;
+  const int r0 = 8 * (wave & 3) + fr;
+  const uint32_t gran = 16u * (uint32_t)(fp ^ frag_swz(r0));
+  const uint32_t w_base = (uint32_t)((int64_t)r0 * p.w_stride) + gran, w_step = (uint32_t)(32 * p.w_stride);
+  const uint32_t x_base = (uint32_t)(r0 * Kc * kFp8Block) + gran, x_step = (uint32_t)(32 * Kc * kFp8Block);
+  const uint32_t row_lds = lds0 + 1024u * (uint32_t)(wave & 3);
+  // A wave's loads: rows 32 i .. of the weight or of the activation tile.
+  // With two buffers waves 0-3 load activations and waves 4-7 weights; with
+  // three each group loads half of a stage, kBoth weight loads and then the
+  // rest of the weights (waves 0-3) or the activations (waves 4-7).
+  constexpr int kX = T::BM / 32, kW = T::BN / 32, kXHalf = kX / 2;  // loads per wave of one group: the tile's rows
+  constexpr int kShare = (kX + kW) / 2, kBoth = S == 2 ? 0 : kW - kShare;
+  const bool own_w = S == 2 ? !first : first;  // whether this wave's loads i >= kBoth are weights
+  const u32x4 rl = own_w ? rw : rx;
+  const uint32_t l_step = own_w ? w_step : x_step;
+  const uint32_t l_base = own_w ? w_base + (uint32_t)kBoth * w_step : x_base;
+  const uint32_t l_lds = row_lds + (own_w ? 4096u * kBoth : (uint32_t)T::kWBytes);
+  // rows of stage kc (past the last stage: bytes that are never read) into buffer buf
+  auto load_rows = [&](int i, int kc, int buf) {
+    dma_load16_keep(rl, l_base + (uint32_t)i * l_step + (uint32_t)kc * kFp8Block,
+                    l_lds + (uint32_t)(buf * T::kStage) + 4096u * (uint32_t)i);
+  };
+  auto load_sx = [&](int i, int kc, int buf) {  // scales of token rows 64 i .. (the dword that holds each)
+    dma_load4_keep(rsx, ((uint32_t)((64 * i + lane) * Kc + kc) * 2u) & ~3u,
+                   lds0 + (uint32_t)(buf * T::kStage + T::kWBytes + T::kXBytes + 256 * i));
+  };
+  const uint32_t sw_lds = lds0 + (uint32_t)(S * T::kStage);
+  for (int i = wave; i < (int)(round_up_1k(((int64_t)T::kWBlocks * Kc + 8) * 2) / 1024); i += T::kWaves)
+    dma_load16_keep(rsw, 1024u * i + 16u * lane, sw_lds + 1024u * i);
+
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int q = lane >> 4, r16 = lane & 15;
+  const uint16_t* sw_rows = reinterpret_cast<const uint16_t*>(smem + S * T::kStage) + sw_shift +
+                            (T::BN <= kFp8Block ? 0 : (wn * TN * 16) / kFp8Block) * Kc;
+  i32x8 a[TN], b[TM];  // all of a K block's fragments: once read, its buffer is free
+  float s[TM];
+  const uint32_t lo16 = (uint32_t)(r16 * kFp8Block + 16 * (q ^ frag_swz(r16)));
+  auto frag = [&](const uint8_t* rows) {  // granules q and q + 4, as read_frag
+    const u32x4 x = *reinterpret_cast<const u32x4*>(rows + lo16), y = *reinterpret_cast<const u32x4*>(rows + (lo16 ^ 64u));
+    return i32x8{(int)x.x, (int)x.y, (int)x.z, (int)x.w, (int)y.x, (int)y.y, (int)y.z, (int)y.w};
+  };
+  // Fragments and scales of K block kc from buffer buf; on return they are in
+  // registers.  At a higher priority: the other wave of the SIMD is in its
+  // MFMAs, and a late read holds up both (1-2 % of a call).
+  auto read = [&](int kc, int buf) {
+    __builtin_amdgcn_s_setprio(2);
+    const uint8_t* st = smem + buf * T::kStage;
+    const uint8_t* wrows = st + (wn * TN * 16) * kFp8Block;
+    const uint8_t* xrows = st + T::kWBytes + (wm * TM * 16) * kFp8Block;
+    const uint32_t* sx_dw = reinterpret_cast<const uint32_t*>(st + T::kWBytes + T::kXBytes);
+    const float sw = bf16_bits_to_f32(sw_rows[kc]);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int row = wm * TM * 16 + 16 * j + r16;
+      const uint32_t d = sx_dw[row];
+      s[j] = bf16_bits_to_f32((row * Kc + kc) & 1 ? d >> 16 : d & 0xFFFFu) * sw;  // exact (two bf16 values)
+      b[j] = frag(xrows + 16 * j * kFp8Block);
+    }
+#pragma unroll
+    for (int i = 0; i < TN; ++i) a[i] = frag(wrows + 16 * i * kFp8Block);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(b[j]), "+v"(s[j]));
+#pragma unroll
+    for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(a[i]));
+    __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0): the buffer may be overwritten
+    __builtin_amdgcn_s_setprio(0);
+  };
+  // MFMA t of a K block: fragment (t / TM, t % TM); its product is added kLag
+  // MFMAs later; hook(t) issues the phase's loads
+  auto compute = [&](auto&& hook) {
+    constexpr int kN = TN * TM, kLag = 3;
+    f32x4 part[kLag + 1];
+#pragma unroll
+    for (int t = 0; t < kN + kLag; ++t) {
+      if (t < kN) {
+        part[t % (kLag + 1)] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+            a[t / TM], b[t % TM], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 127, 0, 127);
+      }
+      if (t >= kLag) {
+        const int u = t - kLag, i = u / TM, j = u % TM;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_fmaf(part[u % (kLag + 1)][e], s[j], acc[i][j][e]);
+        asm volatile("" : "+v"(acc[i][j]));  // here, not sunk past the barrier
+      }
+      if (t < kN) hook(t);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // Both groups run the same steps, waves 4-7 one barrier later: in phase 2 kc
+  // waves 0-3 compute K block kc and waves 4-7 read its fragments, in phase
+  // 2 kc + 1 waves 4-7 compute it and waves 0-3 read those of kc + 1.
+  if constexpr (S == 2) {
+    // The activation rows of the first half are read by waves 0-3 only, the
+    // others by waves 4-7 only, the weights by both.  So waves 0-3 load, in
+    // phase 2 kc, the second half's rows of stage kc + 1 and their own half's
+    // of stage kc + 2 (each half's buffer was last read one phase before),
+    // waves 4-7, in phase 2 kc + 1, the weights of stage kc + 2.
+    static_assert(T::BM == 256, "one scale load per wave 0-3 and K block");
+    constexpr int kN = TN * TM;
+    static_assert(kN >= 4 * kXHalf + 4 && kN >= kW, "loads of a phase");
+    if (first) {
+#pragma unroll
+      for (int i = 0; i < kX; ++i) load_rows(i, 0, 0);
+      load_sx(wave, 0, 0);
+#pragma unroll
+      for (int i = 0; i < kXHalf; ++i) load_rows(i, 1, 1);
+      if (wave < 2) load_sx(wave, 1, 1);
+      wait_vmcnt<kXHalf>();  // stage 0 and the weight scales
+    } else {
+#pragma unroll
+      for (int i = 0; i < kW; ++i) load_rows(i, 0, 0);
+#pragma unroll
+      for (int i = 0; i < kW; ++i) load_rows(i, 1, 1);
+      wait_vmcnt<kW>();
+    }
+    lds_barrier();
+    if (first) {
+      for (int kc = 0; kc < Kc; ++kc) {
+        const int buf = kc & 1;
+        read(kc, buf);
+        if (kc > 0) wait_vmcnt<kXHalf>();  // the other half's rows of stage kc
+        lds_barrier();
+        compute([&](int t) {
+          if (t % 2 == 0 && t / 2 < kXHalf) load_rows(kXHalf + t / 2, kc + 1, buf ^ 1);
+          if (t == 2 * kXHalf) load_sx(wave, kc + 2 - (wave >> 1), (kc - (wave >> 1)) & 1);
+          if (t % 2 == 0 && t / 2 > kXHalf && t / 2 <= 2 * kXHalf) load_rows(t / 2 - kXHalf - 1, kc + 2, buf);
+        });
+        wait_vmcnt<2 * kXHalf + 1>();  // this half's rows of stage kc + 1
+        lds_barrier();
+      }
+      lds_barrier();
+    } else {
+      lds_barrier();
+      for (int kc = 0; kc < Kc; ++kc) {
+        const int buf = kc & 1;
+        read(kc, buf);
+        wait_vmcnt<0>();  // the weights of stage kc + 1
+        lds_barrier();
+        compute([&](int t) {
+          if (t < kW) load_rows(t, kc + 2, buf);
+        });
+        lds_barrier();
+      }
+    }
+  } else {
+    // Three buffers: waves 0-3 load the first half of stage kc + 2 (its buffer
+    // was last read in phase 2 kc - 2), waves 4-7 the second half of stage
+    // kc + 3 (last read in phase 2 kc), each while it computes K block kc.
+    static_assert((kX + kW) % 2 == 0 && kBoth >= 0 && TN * TM >= kShare + 1 && T::BM == 128, "loads of a phase");
+    const uint32_t b_base = w_base + (first ? 0u : (uint32_t)kShare * w_step);
+    const uint32_t b_lds = row_lds + (first ? 0u : 4096u * kShare);
+    auto load_share = [&](int i, int kc, int buf) {  // load i of this group's half of a stage, the scales last
+      if (i < kBoth)
+        dma_load16_keep(rw, b_base + (uint32_t)i * w_step + (uint32_t)kc * kFp8Block,
+                        b_lds + (uint32_t)(buf * T::kStage) + 4096u * (uint32_t)i);
+      else if (i < kShare) load_rows(i - kBoth, kc, buf);
+      else if ((wave & 3) == 0) load_sx(first ? 0 : 1, kc, buf);
+    };
+    auto wait_share = [&] {  // all but the newest share has landed
+      if ((wave & 3) == 0) wait_vmcnt<kShare + 1>();
+      else wait_vmcnt<kShare>();
+    };
+#pragma unroll
+    for (int i = 0; i <= kShare; ++i) load_share(i, 0, 0);
+#pragma unroll
+    for (int i = 0; i <= kShare; ++i) load_share(i, 1, 1);
+    if (!first) {
+#pragma unroll
+      for (int i = 0; i <= kShare; ++i) load_share(i, 2, 2);
+    }
+    // stage 0 (and the weight scales) has landed; wave w & 3 == 0 has one load more per stage, a stricter wait for it
+    if (first) wait_vmcnt<kShare>();
+    else wait_vmcnt<2 * kShare>();
+    lds_barrier();
+    if (!first) lds_barrier();
+    int buf = 0;
+    for (int kc = 0; kc < Kc; ++kc) {
+      read(kc, buf);
+      if (!first) wait_share();  // its half of stage kc + 1 (stage kc + 2 may be in flight)
+      lds_barrier();
+      const int prev = buf == 0 ? 2 : buf - 1;  // (kc + 2) % 3
+      const int to = first ? prev : buf, lk = first ? kc + 2 : kc + 3;
+      compute([&](int t) {
+        if (t <= kShare) load_share(t, lk, to);
+      });
+      if (first) wait_share();  // its half of stage kc + 1
+      lds_barrier();
+      buf = buf == 2 ? 0 : buf + 1;
+    }
+    if (first) lds_barrier();
+  }
+  wait_vmcnt<0>();  // nothing may land in LDS after the workgroup exits
+
+  // out[m][n]: as in the tile kernel
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int64_t m = m0 + wm * TM * 16 + 16 * j + r16;
+    if (m >= p.M) continue;
+    uint16_t* orow = p.out + m * p.out_stride + n0 + wn * TN * 16 + 4 * q;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const f32x4 v = acc[i][j];
+      const u32x2 o = F16_OUT ? u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])}
+                              : u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      *reinterpret_cast<u32x2*>(orow + 16 * i) = o;
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Skinny GEMM (M <= 256 tokens): the weights stream once, into registers
 // ---------------------------------------------------------------------------
@@ -508,26 +786,21 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
   *reinterpret_cast<u32x2*>(out + m * out_stride + n) = o;
 }
 
-// Tile configurations, largest first: (WN, WM, TN, TM) -> BN x BM.
-//   0: 2 x 4 waves, 8 x 4 fragments -> 256 features x 256 tokens (one
-//      workgroup of 8 waves per CU: a K block is ~1 us of MFMA work, about
-//      the latency of the next block's loads, which the second buffer hides)
+// Tile configurations: (WN, WM, TN, TM) -> BN x BM.
+//   0: 2 x 4 waves, 8 x 4 fragments -> 256 features x 256 tokens, two groups in
+//      turn (swap_gemm_kernel), two stages: the fewest bytes per MFMA
 //   1: 2 x 2 waves, 4 x 2 fragments -> 128 x 64
 //   2: 4 x 1 waves, 2 x 2 fragments -> 128 x 32
 //   3: 2 x 1 waves, 2 x 1 fragments ->  64 x 16
-// (A 256 x 128 tile on 4 waves was slower than 1 at every size measured:
-// with one wave per SIMD neither the loads nor the FMAs overlap the MFMAs.)
-// and, outside that order, for 64 < M <= 192 tokens:
-//   4: 2 x 6 waves, 3 x 2 fragments -> 96 x 192 (all the tokens), a ring of 4
-//      stages: a K block of 192 tokens is ~0.1 us of MFMA work per CU, so
-//      with one stage in flight every block waits a full load round trip;
-//      three stages in flight keep the weight stream going, and with N / 96
-//      tiles (a multiple of the CUs for Qwen3-8B gate/up) each weight byte is
-//      read once.
-constexpr int kGemmConfigs = 5;
-constexpr int kGemmOrdered = 4;  // configurations 0 .. 3 form the size order
-constexpr int kGemmBN[kGemmConfigs] = {256, 128, 128, 64, 96};
-constexpr int kGemmBM[kGemmConfigs] = {256, 64, 32, 16, 192};
+//   4: 2 x 6 waves, 3 x 2 fragments -> 96 x 192, a ring of 4 stages, for at
+//      most 192 tokens: all of them in one tile, so with N / 96 tiles (a
+//      multiple of the CUs for Qwen3-8B gate/up) each weight byte is read
+//      once, and three stages in flight keep the weight stream going
+//   5: 4 x 2 waves, 4 x 4 fragments -> 256 x 128, two groups in turn, three
+//      stages, for calls whose 256 x 256 tiles would leave CUs idle
+constexpr int kGemmConfigs = 6;
+constexpr int kGemmBN[kGemmConfigs] = {256, 128, 128, 64, 96, 256};
+constexpr int kGemmBM[kGemmConfigs] = {256, 64, 32, 16, 192, 128};
 
 int64_t config_lds_bytes(int c, int Kc) {
   switch (c) {
@@ -535,7 +808,8 @@ int64_t config_lds_bytes(int c, int Kc) {
     case 1: return gemm_lds_bytes<2, 2, 4, 2>(Kc);
     case 2: return gemm_lds_bytes<4, 1, 2, 2>(Kc);
     case 3: return gemm_lds_bytes<2, 1, 2, 1>(Kc);
-    default: return gemm_lds_bytes<2, 6, 3, 2, 4>(Kc);
+    case 4: return gemm_lds_bytes<2, 6, 3, 2, 4>(Kc);
+    default: return gemm_lds_bytes<4, 2, 4, 4, 3>(Kc);
   }
 }
 
@@ -552,6 +826,23 @@ hipError_t launch_config(const Fp8GemmParams& p, int64_t lds, hipStream_t stream
   }
   const dim3 grid((unsigned)(p.N / T::BN), (unsigned)((p.M + T::BM - 1) / T::BM));
   hipLaunchKernelGGL(kern, grid, dim3(T::kThreads), (size_t)lds, stream, p);
+  return hipGetLastError();
+}
+
+template <int WN, int WM, int TN, int TM, int S, bool F16_OUT>
+hipError_t launch_swap(const Fp8GemmParams& p, int64_t lds, hipStream_t stream) {
+  using T = GemmTile<WN, WM, TN, TM, S>;
+  auto kern = swap_gemm_kernel<WN, WM, TN, TM, S, F16_OUT>;
+  static std::atomic<int64_t> lds_set{0};  // largest dynamic LDS size granted so far
+  if (lds > lds_set.load(std::memory_order_relaxed)) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)lds);
+    if (e != hipSuccess) return e;
+    lds_set.store(lds, std::memory_order_relaxed);
+  }
+  const int64_t tiles = (p.N / T::BN) * ((p.M + T::BM - 1) / T::BM);
+  if (tiles > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(T::kThreads), (size_t)lds, stream, p);
   return hipGetLastError();
 }
 
@@ -628,8 +919,12 @@ SkinnyPlan fp8_skinny_plan(int64_t M, int64_t N, int Kc, int cus, int64_t worksp
   // tokens: gate/up, 576 tiles of 128 x 64, 41.8 us against 50 us here); the
   // small-M kernel is for grids that would leave CUs idle (qkv 144 tiles:
   // 27.3 -> 24.3 us; down 96 tiles: 63.7 -> 35.3 us, weights streamed from
-  // HBM).
+  // HBM).  Nor for short rows, where a K split has nothing to gain (us per
+  // call, tiles against this kernel: 256 tokens on 6,144 x 4,096 29.8 / 37.9,
+  // but 29.5 / 28.1 on 4,096 x 4,096 and 69 / 49 on 4,096 x 12,288; 64 tokens
+  // on 1,024 x 2,048 10.4 / 13.6, 192 tokens 14.9 / 14.3).
   if ((N / 128) * ((M + 63) / 64) >= cus) return best;
+  if (M > 192 ? Kc < 64 && (N > 4096 || N * Kc * kFp8Block <= (4 << 20)) : M <= 128 && N * Kc * kFp8Block <= (4 << 20)) return best;
   const int mf = M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : M <= 128 ? 8 : M <= 192 ? 12 : 16;
   // Estimated time (us): a workgroup's K blocks are latency-bound, about
   // 0.40 + 0.19 CW us each at 192 tokens (less with fewer token fragments),
@@ -695,19 +990,49 @@ hipError_t launch_fp8_act_quant(const void* x, int64_t x_stride, bool f16_in, vo
   return hipGetLastError();
 }
 
+// Estimated time (us) of a product on configuration 0, 1 or 5, from sweeps of
+// 300 to 4,096 tokens over seven Qwen3 projections: a CU takes one large tile
+// at a time, 1.75 (256 x 256) or 1.15 (256 x 128) us per K block with all CUs
+// busy and 1.3 or 0.95 with few, plus 3 to 5 us to fill and drain; 128 x 64
+// tiles share a CU, 0.4 us per K block each.
+static double gemm_estimate(int config, int64_t tiles, int Kc, int cus) {
+  const double x = (double)tiles / cus;
+  if (config == 1) return 1.0 + Kc * std::max(0.85, 0.15 + 0.40 * x);
+  const double full = config == 0 ? 1.75 : 1.15, few = config == 0 ? 1.3 : 0.95;
+  const double whole = std::floor(x), part = x - whole;
+  return (config == 0 ? 3.0 : 5.0) + Kc * (whole * full + (part > 0 ? few + (full - few) * part : 0.0));
+}
+
 int fp8_gemm_pick_config(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit) {
-  // 64 < M <= 192 with whole 96-feature tiles covering the CUs: the deep-ring
-  // tile over all the tokens
-  if (M > 64 && M <= kGemmBM[4] && N % kGemmBN[4] == 0 && N / kGemmBN[4] >= cus &&
-      config_lds_bytes(4, Kc) <= lds_limit)
-    return 4;
-  // the largest tile whose grid still covers the CUs and whose LDS fits;
-  // otherwise the smallest tile that fits
+  auto tiles = [&](int c) { return (N / kGemmBN[c]) * ((M + kGemmBM[c] - 1) / kGemmBM[c]); };
+  auto fits = [&](int c) { return N % kGemmBN[c] == 0 && config_lds_bytes(c, Kc) <= lds_limit; };
+  // 32 < M <= 192 with whole 96-feature tiles covering the CUs (24,576 x
+  // 4,096, us per call: 48 tokens 29.9 against 36.5 on 128 x 64 tiles, 192
+  // tokens 40.2 against 46.6)
+  if (M > 32 && M <= kGemmBM[4] && fits(4) && N / kGemmBN[4] >= cus) return 4;
+  // Enough 128 x 64 tiles for the CUs: the fastest of the three large tiles
+  // by the estimate (us per call; 256 x 256 / 256 x 128 / 128 x 64):
+  // 24,576 x 4,096, M 512: 62.0 / 81.6 / 90.6; 4,096 x 12,288, M 1,888: 146 /
+  // 124 / 162; 4,096 x 4,096, M 1,024: 54.1 / 39.1 / 29.3.
   int best = -1;
-  for (int c = 0; c < kGemmOrdered; ++c) {
-    if (N % kGemmBN[c] != 0 || config_lds_bytes(c, Kc) > lds_limit) continue;
+  if (fits(1) && tiles(1) >= cus) {
+    double best_t = 0.0;
+    for (int c : {1, 5, 0}) {
+      if (!fits(c)) continue;
+      const double t = gemm_estimate(c, tiles(c), Kc, cus);
+      if (best < 0 || t < best_t) {
+        best = c;
+        best_t = t;
+      }
+    }
+    return best;
+  }
+  // otherwise the largest small tile whose grid covers the CUs, or the
+  // smallest that fits
+  for (int c = 0; c <= 3; ++c) {
+    if (!fits(c)) continue;
     best = c;
-    if ((N / kGemmBN[c]) * ((M + kGemmBM[c] - 1) / kGemmBM[c]) >= cus) return c;
+    if (tiles(c) >= cus) return c;
   }
   return best;
 }
@@ -720,8 +1045,8 @@ hipError_t launch_fp8_block_gemm(const Fp8GemmParams& p, int config, bool f16_ou
     return hipErrorInvalidValue;
   const int64_t lds = config_lds_bytes(config, p.Kc);
   switch (config * 2 + (f16_out ? 1 : 0)) {
-    case 0: return launch_config<2, 4, 8, 4, 2, false>(p, lds, stream);
-    case 1: return launch_config<2, 4, 8, 4, 2, true>(p, lds, stream);
+    case 0: return launch_swap<2, 4, 8, 4, 2, false>(p, lds, stream);
+    case 1: return launch_swap<2, 4, 8, 4, 2, true>(p, lds, stream);
     case 2: return launch_config<2, 2, 4, 2, 2, false>(p, lds, stream);
     case 3: return launch_config<2, 2, 4, 2, 2, true>(p, lds, stream);
     case 4: return launch_config<4, 1, 2, 2, 2, false>(p, lds, stream);
@@ -729,7 +1054,9 @@ hipError_t launch_fp8_block_gemm(const Fp8GemmParams& p, int config, bool f16_ou
     case 6: return launch_config<2, 1, 2, 1, 2, false>(p, lds, stream);
     case 7: return launch_config<2, 1, 2, 1, 2, true>(p, lds, stream);
     case 8: return launch_config<2, 6, 3, 2, 4, false>(p, lds, stream);
-    default: return launch_config<2, 6, 3, 2, 4, true>(p, lds, stream);
+    case 9: return launch_config<2, 6, 3, 2, 4, true>(p, lds, stream);
+    case 10: return launch_swap<4, 2, 4, 4, 3, false>(p, lds, stream);
+    default: return launch_swap<4, 2, 4, 4, 3, true>(p, lds, stream);
   }
 }
 

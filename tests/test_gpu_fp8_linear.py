@@ -363,3 +363,30 @@ def test_act_quant_edge_groups(dtype):
     torch.cuda.synchronize()
     assert np.array_equal(xq.cpu().numpy(), xq_ref)
     assert np.array_equal(_bits(xs), xs_ref)
+
+
+@pytest.mark.parametrize("M,N,K", [(4001, 4096, 128), (4096, 4096, 256), (3850, 4096, 384), (8000, 2048, 1152),
+                                   (1889, 4096, 128), (1900, 4096, 256), (2048, 4096, 384), (1800, 4096, 512),
+                                   (1793, 4096, 1152)])
+def test_group_swap_tiles(M, N, K):
+    """The 256 x 256 and 256 x 128 tiles whose two wave groups take turns, from
+    one K block (the prologue's loads only) over the ring's depth to more,
+    with a ragged last tile; against the block-scaled sum in torch fp32."""
+    announce(f"fp8 linear: GEMM {M} x {N} x {K}, wave groups in turn")
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    xq = torch.randint(0, 256, (M, K), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    w = torch.randint(0, 256, (N, K), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    xq, w = (torch.where((c & 0x7F) == 0x7F, c ^ 0x01, c) for c in (xq, w))
+    x_scale = (torch.rand(M, K // 128, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    w_scale = (torch.rand(N // 128, K // 128, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    got = _gemm_gpu(xq, x_scale, w, w_scale).cuda().double()
+    t = torch.from_numpy(fp8.dequant_table().astype(np.float32)).cuda()
+    xd, wd = t[xq.long()], t[w.long()]
+    acc, absum = torch.zeros(M, N, device="cuda"), torch.zeros(M, N, device="cuda")
+    for kc in range(K // 128):
+        xb, wb = xd[:, 128 * kc:128 * (kc + 1)], wd[:, 128 * kc:128 * (kc + 1)].T.contiguous()
+        s = x_scale[:, kc:kc + 1].float() * w_scale[:, kc].float().repeat_interleave(128)[None, :]
+        acc += torch.matmul(xb, wb) * s
+        absum += torch.matmul(xb.abs(), wb.abs()) * s
+    bad = (got - acc.double()).abs() > 2.0 ** -7 * acc.double().abs() + ABS_TOL * absum.double()
+    assert not bad.any(), f"{int(bad.sum())} outputs off, first at {bad.nonzero()[0].tolist()}"
