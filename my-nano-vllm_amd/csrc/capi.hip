@@ -315,7 +315,7 @@ int32_t nvamd_fp8_act_quant(const void* x, int64_t x_stride0, int32_t x_dtype, v
   if ((uintptr_t)x % 16 != 0 || x_stride0 % 8 != 0 || (uintptr_t)xq % 8 != 0 || (uintptr_t)x_scale % 2 != 0)
     return fail(NVAMD_ERR_UNSUPPORTED, "%s: x must be 16-byte aligned with a row stride of 8 elements (xq 8-byte aligned)",
                 fn);
-  return launch_status(nvamd::launch_fp8_act_quant(x, x_stride0, x_dtype == NVAMD_DTYPE_F16, xq, x_scale, M, K,
+  return launch_status(nvamd::launch_fp8_act_quant(x, x_stride0, x_dtype == NVAMD_DTYPE_F16, xq, x_scale, M, K, false,
                                                    (hipStream_t)stream),
                        fn);
 }
@@ -383,6 +383,10 @@ nvamd::Fp8GemmParams gemm_params(const void* xq, const void* x_scale, const void
   p.N = (int)N;
   p.K = (int)K;
   p.Kc = (int)(K / 128);
+  p.x_row = (uint32_t)K;
+  p.x_blk = 128;
+  p.sx_row = (uint32_t)p.Kc;
+  p.sx_blk = 1;
   return p;
 }
 
@@ -451,7 +455,18 @@ int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   p.xq = ws;
   p.x_scale = reinterpret_cast<const uint16_t*>(ws + align_up(M * K));
-  if (int32_t e = nvamd_fp8_act_quant(x, x_stride0, x_dtype, ws, ws + align_up(M * K), M, K, stream)) return e;
+  if (M * K < (1ll << 31) && K <= 128ll * 16 * 0xffff) {
+    // quantised activations by K block: the GEMM's tile loads are contiguous
+    p.x_row = 128;
+    p.x_blk = (uint32_t)(M * 128);
+    p.sx_row = 1;
+    p.sx_blk = (uint32_t)M;
+    const hipError_t e = nvamd::launch_fp8_act_quant(x, x_stride0, f16, ws, ws + align_up(M * K), M, K, true,
+                                                     (hipStream_t)stream);
+    if (e != hipSuccess) return launch_status(e, fn);
+  } else if (int32_t e = nvamd_fp8_act_quant(x, x_stride0, x_dtype, ws, ws + align_up(M * K), M, K, stream)) {
+    return e;
+  }
   const int64_t left = workspace_bytes - act;
   return run_block_gemm(fn, p, f16, left > 0 ? ws + act : nullptr, left, (hipStream_t)stream);
 }

@@ -54,20 +54,28 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 // Dynamic activation quantisation
 // ---------------------------------------------------------------------------
 // Grid (M, ceil(Kc / 16)): workgroup (m, y) quantises groups 16 y .. 16 y + 15
-// of token m, one 16-lane group each, so no lane divides.
+// of token m, one 16-lane group each, so no lane divides and the workgroup
+// reads 4 KiB in one piece.  Where they go: token m's bytes of group g at
+// m * x_row + g * x_blk, its scale at m * sx_row + g * sx_blk, by row or by K
+// block (see Fp8GemmParams).  By K block the GEMM's loads of a tile's rows in
+// one block are contiguous (rows of K bytes put them on a few L2 channels when
+// K is a power of two) and those of its scales 128 bytes instead of 64 lines:
+// its kernel at 1,888 tokens x 12,288 -> 4,096 109 -> 102 us, at 192 tokens x
+// 4,096 -> 24,576 37.0 -> 34.9 us; this kernel takes the same time (14.3 and
+// 14.6 us at 1,888 x 12,288).  Workgroups of 2 or 4 tokens, or of 16 tokens and
+// 4 groups with four loads in flight per lane, were 3-40 % slower.
 template <bool F16_IN>
 __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
-                                                        uint8_t* __restrict__ xq, uint16_t* __restrict__ x_scale,
-                                                        int64_t M, int Kc) {
+                                                        uint8_t* __restrict__ xq, uint16_t* __restrict__ x_scale, int Kc,
+                                                        int64_t x_row, int64_t x_blk, int64_t sx_row, int64_t sx_blk) {
   const int64_t m = blockIdx.x;
   const int g = 16 * (int)blockIdx.y + (int)(threadIdx.x >> 4);  // 128-column group of the token
   const int j = (int)(threadIdx.x & 15);
   if (g >= Kc) return;  // whole 16-lane groups
   const u32x4 w = *reinterpret_cast<const u32x4*>(x + m * x_stride + (int64_t)g * kFp8Block + 8 * j);
   float scale;
-  *reinterpret_cast<u32x2*>(xq + m * ((int64_t)Kc * kFp8Block) + (int64_t)g * kFp8Block + 8 * j) =
-      quant_group8<F16_IN>(w, scale);
-  if (j == 0) x_scale[m * Kc + g] = (uint16_t)scale_bf16_bits(scale);
+  *reinterpret_cast<u32x2*>(xq + m * x_row + g * x_blk + 8 * j) = quant_group8<F16_IN>(w, scale);
+  if (j == 0) x_scale[m * sx_row + g * sx_blk] = (uint16_t)scale_bf16_bits(scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -107,6 +115,17 @@ template <int WN, int WM, int TN, int TM, int S = 2>
 constexpr int64_t gemm_scale_offset() { return (int64_t)S * GemmTile<WN, WM, TN, TM, S>::kStage; }
 
 __host__ __device__ constexpr int64_t round_up_1k(int64_t b) { return (b + 1023) & ~(int64_t)1023; }
+
+// Bytes of the activations and of their scales from the first of `rows` token
+// rows on.  Scale descriptors end on a whole dword: the bounds check drops a
+// dword that is only partly in range, and an aligned dword never crosses a
+// page.
+__device__ __forceinline__ uint32_t x_bytes(const Fp8GemmParams& p, int rows) {
+  return (uint32_t)(rows - 1) * p.x_row + (uint32_t)(p.Kc - 1) * p.x_blk + (uint32_t)kFp8Block;
+}
+__device__ __forceinline__ uint32_t sx_bytes(const Fp8GemmParams& p, int rows) {
+  return (((uint32_t)(rows - 1) * p.sx_row + (uint32_t)(p.Kc - 1) * p.sx_blk + 1u) * 2u + 3u) & ~3u;
+}
 
 // LDS bytes of a launch: S stages (weight tile, activation tile, and per
 // token row the dword of x_scale that holds its scale for the K block), then
@@ -155,13 +174,11 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
   const int Kc = p.Kc;
   const int rows_x = (int)min((int64_t)T::BM, p.M - m0);  // valid token rows of the tile
 
-  // descriptors: rows past the matrix (tokens >= M) read as zeros
+  // descriptors: rows past the matrix (tokens >= M) read zeros or, with the
+  // activations by K block, the next block's rows (their columns are not stored)
   const u32x4 rw = rsrc_words(p.w + (int64_t)n0 * p.w_stride, (uint32_t)((int64_t)T::BN * p.w_stride));
-  const u32x4 rx = rsrc_words(p.xq + m0 * ((int64_t)Kc * kFp8Block), (uint32_t)((int64_t)rows_x * Kc * kFp8Block));
-  // scale descriptors end on a whole dword: the bounds check drops a dword
-  // that is only partly in range, and an aligned dword never crosses a page
-  const int64_t sx_bytes = ((int64_t)rows_x * Kc * 2 + 3) & ~(int64_t)3;
-  const u32x4 rsx = rsrc_words(p.x_scale + m0 * Kc, (uint32_t)sx_bytes);
+  const u32x4 rx = rsrc_words(p.xq + m0 * p.x_row, x_bytes(p, rows_x));
+  const u32x4 rsx = rsrc_words(p.x_scale + m0 * p.sx_row, sx_bytes(p, rows_x));
   // weight scales from a 16-byte aligned element (sw_shift elements before the tile's first)
   const int64_t sw_first = (int64_t)(n0 / kFp8Block) * Kc;
   const int sw_shift = (int)(sw_first & 7);
@@ -180,10 +197,10 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
   };
   auto x_off = [&](int i, int kc) {
     const int r = 8 * (wave + T::kWaves * i) + fr;
-    return (uint32_t)((int64_t)r * Kc * kFp8Block + kc * kFp8Block + 16 * (fp ^ frag_swz(r)));
+    return (uint32_t)r * p.x_row + (uint32_t)kc * p.x_blk + (uint32_t)(16 * (fp ^ frag_swz(r)));
   };
   // wave w < kSxLoads: token rows 64 w + lane, the dword holding x_scale[row][kc]
-  const uint32_t sx_row_off = (uint32_t)((64 * wave + lane) * Kc) * 2u;
+  const uint32_t sx_row_off = (uint32_t)(64 * wave + lane) * p.sx_row * 2u;
   auto issue_stage = [&](int kc, int buf) {
     const uint32_t base = lds0 + (uint32_t)(buf * T::kStage);
 #pragma unroll
@@ -198,7 +215,7 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
     for (int i = 0; i < T::kXLoads; ++i)
       dma_load16_keep(rx, x_off(i, kc), base + (uint32_t)(T::kWBytes + 1024 * (wave + T::kWaves * i)));
     if (wave < T::kSxLoads)
-      dma_load4_keep(rsx, (sx_row_off + 2u * kc) & ~3u, base + (uint32_t)(T::kWBytes + T::kXBytes + 256 * wave));
+      dma_load4_keep(rsx, (sx_row_off + 2u * p.sx_blk * (uint32_t)kc) & ~3u, base + (uint32_t)(T::kWBytes + T::kXBytes + 256 * wave));
   };
 
   // weight scales [kWBlocks x Kc], loaded once
@@ -248,7 +265,7 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
     for (int j = 0; j < TM; ++j) {
       const int row = wm * TM * 16 + 16 * j + r16;
       const uint32_t d = sx_dw[row];
-      sx[j] = bf16_bits_to_f32((row * Kc + kc) & 1 ? d >> 16 : d & 0xFFFFu);
+      sx[j] = bf16_bits_to_f32(((uint32_t)row * p.sx_row + (uint32_t)kc * p.sx_blk) & 1u ? d >> 16 : d & 0xFFFFu);
       b[j] = read_frag(xrows + 16 * j * kFp8Block, r16, q);
     }
     float s[TM];
@@ -339,9 +356,8 @@ __global__ __launch_bounds__(512) void swap_gemm_kernel(Fp8GemmParams p) {
 
   // descriptors as in the tile kernel
   const u32x4 rw = rsrc_words(p.w + (int64_t)n0 * p.w_stride, (uint32_t)((int64_t)T::BN * p.w_stride));
-  const u32x4 rx = rsrc_words(p.xq + m0 * ((int64_t)Kc * kFp8Block), (uint32_t)((int64_t)rows_x * Kc * kFp8Block));
-  const int64_t sx_bytes = ((int64_t)rows_x * Kc * 2 + 3) & ~(int64_t)3;
-  const u32x4 rsx = rsrc_words(p.x_scale + m0 * Kc, (uint32_t)sx_bytes);
+  const u32x4 rx = rsrc_words(p.xq + m0 * p.x_row, x_bytes(p, rows_x));
+  const u32x4 rsx = rsrc_words(p.x_scale + m0 * p.sx_row, sx_bytes(p, rows_x));
   const int64_t sw_first = (int64_t)(n0 / kFp8Block) * Kc;
   const int sw_shift = (int)(sw_first & 7);
   const int64_t sw_elems = (int64_t)T::kWBlocks * Kc + sw_shift;
@@ -354,7 +370,7 @@ __global__ __launch_bounds__(512) void swap_gemm_kernel(Fp8GemmParams p) {
   const int r0 = 8 * (wave & 3) + fr;
   const uint32_t gran = 16u * (uint32_t)(fp ^ frag_swz(r0));
   const uint32_t w_base = (uint32_t)((int64_t)r0 * p.w_stride) + gran, w_step = (uint32_t)(32 * p.w_stride);
-  const uint32_t x_base = (uint32_t)(r0 * Kc * kFp8Block) + gran, x_step = (uint32_t)(32 * Kc * kFp8Block);
+  const uint32_t x_base = (uint32_t)r0 * p.x_row + gran, x_step = 32u * p.x_row;
   const uint32_t row_lds = lds0 + 1024u * (uint32_t)(wave & 3);
   // A wave's loads: rows 32 i .. of the weight or of the activation tile.
   // With two buffers waves 0-3 load activations and waves 4-7 weights; with
@@ -364,16 +380,16 @@ __global__ __launch_bounds__(512) void swap_gemm_kernel(Fp8GemmParams p) {
   constexpr int kShare = (kX + kW) / 2, kBoth = S == 2 ? 0 : kW - kShare;
   const bool own_w = S == 2 ? !first : first;  // whether this wave's loads i >= kBoth are weights
   const u32x4 rl = own_w ? rw : rx;
-  const uint32_t l_step = own_w ? w_step : x_step;
+  const uint32_t l_step = own_w ? w_step : x_step, l_blk = own_w ? (uint32_t)kFp8Block : p.x_blk;
   const uint32_t l_base = own_w ? w_base + (uint32_t)kBoth * w_step : x_base;
   const uint32_t l_lds = row_lds + (own_w ? 4096u * kBoth : (uint32_t)T::kWBytes);
   // rows of stage kc (past the last stage: bytes that are never read) into buffer buf
   auto load_rows = [&](int i, int kc, int buf) {
-    dma_load16_keep(rl, l_base + (uint32_t)i * l_step + (uint32_t)kc * kFp8Block,
+    dma_load16_keep(rl, l_base + (uint32_t)i * l_step + (uint32_t)kc * l_blk,
                     l_lds + (uint32_t)(buf * T::kStage) + 4096u * (uint32_t)i);
   };
   auto load_sx = [&](int i, int kc, int buf) {  // scales of token rows 64 i .. (the dword that holds each)
-    dma_load4_keep(rsx, ((uint32_t)((64 * i + lane) * Kc + kc) * 2u) & ~3u,
+    dma_load4_keep(rsx, (((uint32_t)(64 * i + lane) * p.sx_row + (uint32_t)kc * p.sx_blk) * 2u) & ~3u,
                    lds0 + (uint32_t)(buf * T::kStage + T::kWBytes + T::kXBytes + 256 * i));
   };
   const uint32_t sw_lds = lds0 + (uint32_t)(S * T::kStage);
@@ -406,11 +422,12 @@ __global__ __launch_bounds__(512) void swap_gemm_kernel(Fp8GemmParams p) {
     const uint8_t* xrows = st + T::kWBytes + (wm * TM * 16) * kFp8Block;
     const uint32_t* sx_dw = reinterpret_cast<const uint32_t*>(st + T::kWBytes + T::kXBytes);
     const float sw = bf16_bits_to_f32(sw_rows[kc]);
+    // which half of its dword a token's scale is (the same in all fragments: they are 16 rows apart)
+    const uint32_t sh = 16u * (((uint32_t)r16 * p.sx_row + (uint32_t)kc * p.sx_blk) & 1u);
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
-      const int row = wm * TM * 16 + 16 * j + r16;
-      const uint32_t d = sx_dw[row];
-      s[j] = bf16_bits_to_f32((row * Kc + kc) & 1 ? d >> 16 : d & 0xFFFFu) * sw;  // exact (two bf16 values)
+      const uint32_t d = sx_dw[wm * TM * 16 + 16 * j + r16];
+      s[j] = __builtin_bit_cast(float, (d >> sh) << 16) * sw;  // exact (two bf16 values)
       b[j] = frag(xrows + 16 * j * kFp8Block);
     }
 #pragma unroll
@@ -641,8 +658,8 @@ __global__ __launch_bounds__((64 * Skinny<CW, MF>::kWaves)) void skinny_gemm_ker
   if (wave >= CW) {
     // ---- loader waves ------------------------------------------------------
     const int l = wave - CW;
-    const u32x4 rx = rsrc_words(p.xq, (uint32_t)(p.M * p.K));
-    const u32x4 rsx = rsrc_words(p.x_scale, (uint32_t)((p.M * Kc * 2 + 3) & ~3ll));
+    const u32x4 rx = rsrc_words(p.xq, x_bytes(p, (int)p.M));
+    const u32x4 rsx = rsrc_words(p.x_scale, sx_bytes(p, (int)p.M));
     if (l == 0) {
       const u32x4 rsw = rsrc_words(p.w_scale + (sw_first - sw_shift), (uint32_t)(((int64_t)nk + sw_shift) * 2 + 3) & ~3u);
       for (int i = 0; i < (int)(round_up_1k(((int64_t)kper + 8) * 2) / 1024); ++i)
@@ -657,14 +674,14 @@ __global__ __launch_bounds__((64 * Skinny<CW, MF>::kWaves)) void skinny_gemm_ker
       for (int i0 = 0; i0 < T::kXLoads; i0 += T::LW) {
         const int i = i0 + l;
         const int r = 8 * i + fr;
-        dma_load16_keep(rx, (uint32_t)r * (uint32_t)p.K + (uint32_t)kc * kFp8Block + 16u * (uint32_t)(fp ^ frag_swz(r)),
+        dma_load16_keep(rx, (uint32_t)r * p.x_row + (uint32_t)kc * p.x_blk + 16u * (uint32_t)(fp ^ frag_swz(r)),
                         base + 1024u * i);
       }
       if (l == 0) {
 #pragma unroll
         for (int i = 0; i < T::kSxLoads; ++i) {
           const int r = 64 * i + lane;
-          dma_load4_keep(rsx, ((uint32_t)(r * Kc + kc) * 2u) & ~3u, base + (uint32_t)(T::kXBytes + 256 * i));
+          dma_load4_keep(rsx, (((uint32_t)r * p.sx_row + (uint32_t)kc * p.sx_blk) * 2u) & ~3u, base + (uint32_t)(T::kXBytes + 256 * i));
         }
       }
     };
@@ -728,7 +745,7 @@ __global__ __launch_bounds__((64 * Skinny<CW, MF>::kWaves)) void skinny_gemm_ker
       for (int j = 0; j < MF; ++j) {
         const int row = 16 * j + r16;
         const uint32_t d = sx_dw[row];
-        const float s = bf16_bits_to_f32((row * Kc + kc) & 1 ? d >> 16 : d & 0xFFFFu) * sw;  // exact
+        const float s = bf16_bits_to_f32(((uint32_t)row * p.sx_row + (uint32_t)kc * p.sx_blk) & 1u ? d >> 16 : d & 0xFFFFu) * sw;  // exact
         const i32x8 b = read_frag(st + 16 * j * kFp8Block, r16, q);
         const f32x4 pr = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0,
                                                                           127, 0, 127);
@@ -976,17 +993,16 @@ hipError_t launch_fp8_skinny_gemm(const Fp8GemmParams& p, const SkinnyPlan& plan
 }
 
 hipError_t launch_fp8_act_quant(const void* x, int64_t x_stride, bool f16_in, void* xq, void* x_scale, int64_t M,
-                                int64_t K, hipStream_t stream) {
+                                int64_t K, bool by_block, hipStream_t stream) {
   if (M == 0) return hipSuccess;
-  const int64_t ys = (K / kFp8Block + 15) / 16;
+  const int Kc = (int)(K / kFp8Block);
+  const int64_t ys = ((int64_t)Kc + 15) / 16;
   if (M > 0x7fffffff || ys > 0xffff) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)M, (unsigned)ys);
-  if (f16_in)
-    hipLaunchKernelGGL(act_quant_kernel<true>, grid, dim3(256), 0, stream, (const uint16_t*)x, x_stride, (uint8_t*)xq,
-                       (uint16_t*)x_scale, M, (int)(K / kFp8Block));
-  else
-    hipLaunchKernelGGL(act_quant_kernel<false>, grid, dim3(256), 0, stream, (const uint16_t*)x, x_stride,
-                       (uint8_t*)xq, (uint16_t*)x_scale, M, (int)(K / kFp8Block));
+  const int64_t x_row = by_block ? kFp8Block : K, x_blk = by_block ? M * kFp8Block : kFp8Block;
+  const int64_t sx_row = by_block ? 1 : Kc, sx_blk = by_block ? M : 1;
+  auto kern = f16_in ? act_quant_kernel<true> : act_quant_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)M, (unsigned)ys), dim3(256), 0, stream, (const uint16_t*)x, x_stride,
+                     (uint8_t*)xq, (uint16_t*)x_scale, Kc, x_row, x_blk, sx_row, sx_blk);
   return hipGetLastError();
 }
 

@@ -79,29 +79,32 @@ __global__ __launch_bounds__(64 * kThinMaxWaves) void thin_linear_kernel(Fp8Gemm
   // together (two values of q) hit 32 different granules of a 512-byte window.
   const uint32_t rd0 = (uint32_t)(r16 * kThinChunk + 16 * (q ^ (2 * r16)));
 
-  const __amdgpu_buffer_rsrc_t rxq = make_rsrc(p.xq, (uint32_t)(p.M * p.K));
-  const __amdgpu_buffer_rsrc_t rsx = make_rsrc(p.x_scale, (uint32_t)(p.M * Kc * 2));
+  const __amdgpu_buffer_rsrc_t rxq =
+      make_rsrc(p.xq, (uint32_t)(M - 1) * p.x_row + (uint32_t)(Kc - 1) * p.x_blk + (uint32_t)kFp8Block);
+  const __amdgpu_buffer_rsrc_t rsx =
+      make_rsrc(p.x_scale, ((uint32_t)(M - 1) * p.sx_row + (uint32_t)(Kc - 1) * p.sx_blk + 1u) * 2u);
   uint8_t* xs = smem + nw * kThinSlot + wave * thin_x_bytes(M);
   float* ss = reinterpret_cast<float*>(xs + M * kThinXPitch);
 
   u32x4 xr[XI > 0 ? XI : 1], xb[XI > 0 ? 1 : kThinKb][MF][2];
   uint32_t sx2[MF];  // lane (q, token): scales of the chunk's K blocks 2q (low half) and 2q + 1
-  auto load_x = [&](int d, int kc) {  // quantised rows of K block kc, in the operand layout; rows past M read zeros
+  auto load_x = [&](int d, int kc) {  // quantised rows of K block kc, in the operand layout
 #pragma unroll
     for (int j = 0; j < MF; ++j) {
       const uint32_t row = (uint32_t)(16 * j + r16);
-      const bool in = kc < Kc;
-      const uint32_t off = row * (uint32_t)p.K + (uint32_t)kc * kFp8Block + 16u * (uint32_t)q;
+      const bool in = kc < Kc && row < (uint32_t)M;  // rows past M: no traffic
+      const uint32_t off = row * p.x_row + (uint32_t)kc * p.x_blk + 16u * (uint32_t)q;
       xb[d][j][0] = buf_load16(rxq, in ? off : kOutOfRange);
       xb[d][j][1] = buf_load16(rxq, in ? off + 64u : kOutOfRange);
     }
   };
-  auto load_sx = [&](int kc0) {  // (blocks past K: P is 0, and the scale read instead is another row's or 0)
+  auto load_sx = [&](int kc0) {  // (blocks past K: P is 0, and the row's last scale stands in)
+    const uint32_t k0 = (uint32_t)min(kc0 + 2 * q, Kc - 1) * p.sx_blk, k1 = (uint32_t)min(kc0 + 2 * q + 1, Kc - 1) * p.sx_blk;
 #pragma unroll
     for (int j = 0; j < MF; ++j) {
-      const uint32_t off = ((uint32_t)(16 * j + r16) * (uint32_t)Kc + (uint32_t)(kc0 + 2 * q)) * 2u;
-      sx2[j] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsx, (int)off, 0, 0) |
-               ((uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsx, (int)(off + 2u), 0, 0) << 16);
+      const uint32_t row = (uint32_t)(16 * j + r16) * p.sx_row;
+      sx2[j] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsx, (int)((row + k0) * 2u), 0, 0) |
+               ((uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsx, (int)((row + k1) * 2u), 0, 0) << 16);
     }
   };
 

@@ -142,18 +142,21 @@ hipError_t launch_sample_group(const void* logits, int dtype, int64_t stride, in
 
 // FP8 block-scaled linear (128 x 128 weight blocks, 128-wide activation groups).
 struct Fp8GemmParams {
-  const uint8_t* xq;        // E4M3FN [M, K], row stride K
-  const uint16_t* x_scale;  // bf16 [M, K / 128]
+  const uint8_t* xq;        // E4M3FN: token row m's 128 bytes of K block g at m * x_row + g * x_blk
+  const uint16_t* x_scale;  // bf16: its scale at element m * sx_row + g * sx_blk
   const uint8_t* w;         // E4M3FN [N, K], row stride w_stride (bytes)
   const uint16_t* w_scale;  // bf16 [N / 128, K / 128]
   uint16_t* out;            // bf16 or fp16 [M, N], row stride out_stride (elements)
   int64_t w_stride, out_stride;
   int64_t M;
   int N, K, Kc;
+  // by row ([M, K] and [M, K / 128]) or by K block ([K / 128, M, 128] and
+  // [K / 128, M], the linear layer's own scratch)
+  uint32_t x_row, x_blk, sx_row, sx_blk;
 };
 
 hipError_t launch_fp8_act_quant(const void* x, int64_t x_stride, bool f16_in, void* xq, void* x_scale, int64_t M,
-                                int64_t K, hipStream_t stream);
+                                int64_t K, bool by_block, hipStream_t stream);
 // Tile configuration for an M x N x K GEMM on `cus` CUs (-1: none fits lds_limit).
 int fp8_gemm_pick_config(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit);
 int64_t fp8_gemm_lds_bytes(int config, int Kc);
