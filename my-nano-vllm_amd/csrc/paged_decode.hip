@@ -1030,7 +1030,7 @@ __global__ __launch_bounds__(256) void decode_sk_merge_heads_kernel(MqParams p) 
 // Few pairs: a workgroup of kSkWideWaves waves per (sequence, kv head, four
 // query columns), the contributors dealt over the waves.
 constexpr int kSkWideWaves = 8;
-constexpr int64_t kSkWideMaxWgs = 1024;
+constexpr int64_t kSkWideMaxWgs = 1024;  // four a CU
 __global__ __launch_bounds__(64 * kSkWideWaves) void decode_sk_merge_wide_kernel(MqParams p, int groups) {
   __shared__ float sm[kSkWideWaves * 640];
   // 32-bit index: the launch takes this kernel for at most kSkWideMaxWgs workgroups
@@ -1114,17 +1114,19 @@ hipError_t launch_decode_sk(const MqParams& p, int ncb, bool merge, const Prefil
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (!merge) return hipSuccess;  // the caller's next launch merges
-  // Few pairs (at most kSkWideMaxWgs workgroups, four a CU): a pair may be cut
-  // into as many ranges as there are workgroups, and one wave adding them in
-  // turn is a chain of up to W / 8 memory round trips (one 131,072-token
-  // sequence on 32 / 8 heads: 80.8 us per call with one wave a pair, 53.1 with
-  // eight; 8 sequences of 256-4,096: 24.2 and 18.4).
+  // Few pairs: a pair is then cut into more ranges on average (W / pairs) than
+  // one wave adds in one memory round trip (8, or 16 for one row and head per
+  // wave), and a long one into up to W, a chain of up to W / 8 round trips (one
+  // 131,072-token sequence on 32 / 8 heads: 80.8 us per call with one wave a
+  // pair, 53.1 with eight; 8 sequences of 256-4,096: 24.2 and 18.4; but 32
+  // long ones on 64 / 8 heads: 5.2 us of merge with one wave, 6.3 with eight).
+  const bool heads_at_once = !varlen && p.G <= 4;
   const int groups = (p.G * p.mq_max_q + 3) / 4;  // of four query columns
   const int64_t wide_wgs = (int64_t)p.num_seqs * p.Hkv * groups;
-  if (wide_wgs <= kSkWideMaxWgs)
+  if (wide_wgs <= kSkWideMaxWgs && (int64_t)p.num_seqs * (p.Hkv / hg) * (heads_at_once ? 8 : 16) <= p.sk_wgs)
     hipLaunchKernelGGL(decode_sk_merge_wide_kernel, dim3((unsigned)wide_wgs), dim3(64 * kSkWideWaves), 0, stream, p,
                        groups);
-  else if (!varlen && p.G <= 4)
+  else if (heads_at_once)
     hipLaunchKernelGGL(decode_sk_merge_heads_kernel, dim3((unsigned)(((int64_t)p.num_seqs * p.Hkv + 3) / 4)),
                        dim3(256), 0, stream, p);
   else
