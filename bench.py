@@ -894,7 +894,8 @@ def main():
                 + f"); hipBLASLt per-tensor {r['hipblaslt_per_tensor_us']} us")
         extra["fp8_linear"] = dict(
             workload="FP8 block-scaled linear (128x128 weight blocks), Qwen3-8B shapes",
-            kernels="block_gemm_kernel; skinny_gemm_kernel (+ skinny_reduce_kernel when K is split) for at most "
+            kernels="swap_gemm_kernel (large tiles), block_gemm_kernel; thin_linear_kernel for at most 32 tokens; "
+                    "skinny_gemm_kernel (+ skinny_reduce_kernel when K is split) for at most "
                     "256 tokens where the tile grid would leave CUs idle; act_quant_kernel timed separately; "
                     "hipblaslt_per_tensor_us: torch._scaled_mm with one scale per tensor, same operands; weights "
                     "cycled over > 600 MiB (streamed from HBM)", **lin)

@@ -4,13 +4,13 @@
 arguments, assertions and return value (fp8_linear.py:93-139), so
 nanovllm/layers/linear.py (LinearBase.apply_linear, :56-62) can import it
 unchanged.  It is one dispatcher call of the C++ operator
-torch.ops.nvamd.fp8_block_linear (csrc/torch_ops.cpp), which runs the
-reference's two steps as two hand-written HIP kernels behind the C ABI in
-include/nvamd_fp8_linear.h, enqueued on torch's current stream: the
-per-token, per-128-column dynamic activation quantisation
-(``nvamd_fp8_act_quant``) and the 128 x 128 block-scaled FP8 GEMM
-(``nvamd_fp8_block_gemm``).  The quantised activations and their scales are
-allocated from torch's caching allocator, like the reference's.
+torch.ops.nvamd.fp8_block_linear (csrc/torch_ops.cpp), one call of
+``nvamd_fp8_block_linear`` behind the C ABI in include/nvamd_fp8_linear.h,
+enqueued on torch's current stream: the per-token, per-128-column dynamic
+activation quantisation and the 128 x 128 block-scaled FP8 GEMM as hand-written
+HIP kernels (one kernel for a few tokens).  Scratch for the quantised
+activations and their scales comes from torch's caching allocator, like the
+reference's.
 
 There is no Triton and no CPU fallback: tensors must live on a ROCm GPU and
 the native libraries must be built, otherwise the call raises.

@@ -15,15 +15,14 @@ largest error seen is 2^-15 of the sum of absolute terms; a misplaced or
 missing K block errs by about 2^-3.5 of it.
 
 Shapes are chosen so that on a 256-CU MI355X the library picks each of its
-tile shapes (256x256, 128x64, 128x32, 64x16 features x tokens): it takes the
-largest tile whose grid still covers the CUs.  65 to 192 tokens with at least
-a CU's worth of 96-feature tiles take the 96x192 tile with a 4-stage ring
-(tiles straddle the 128-row weight blocks, so fragments take their own
-scales; K shorter than the ring).  Products with at most 256 tokens whose tile
-grid would leave CUs idle take the small-M kernel instead (weights streamed
-once; K split over workgroups with fp32 partials added in split order when the
-workspace allows): its cases cover 1 to 256 tokens, 2, 4 and 8 compute waves,
-splits and no workspace.
+kernels: the 256x256 and 256x128 tiles whose two wave groups take turns, the
+128x64, 128x32 and 64x16 tiles (features x tokens), the 96x192 tile with a
+4-stage ring for 33 to 192 tokens with at least a CU's worth of 96-feature tiles
+(tiles straddle the 128-row weight blocks, so fragments take their own scales;
+K shorter than the ring), the small-M kernel for products of at most 256 tokens
+whose tile grid would leave CUs idle (K split over workgroups with fp32 partials
+added in split order when the workspace allows), and the kernel for at most 32
+tokens that streams the weights without barriers.
 """
 import numpy as np
 import pytest
