@@ -91,6 +91,24 @@ int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype
  * current device (0: none). */
 int64_t nvamd_fp8_block_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
+/*
+ * The kernel an M x N x K product takes on the current device, given the
+ * workspace it asks for: on quantised activations (quantised != 0, as
+ * nvamd_fp8_block_gemm) or as the whole layer.  Host logic only (no device:
+ * that of an MI355X).  *lds_bytes (may be NULL) receives the LDS of one
+ * workgroup.  NVAMD_LINEAR_* or -1 (bad sizes, or no tile's scales fit).
+ */
+#define NVAMD_LINEAR_TILE_256X256 0 /* features x tokens, two wave groups in turn */
+#define NVAMD_LINEAR_TILE_128X64 1
+#define NVAMD_LINEAR_TILE_128X32 2
+#define NVAMD_LINEAR_TILE_64X16 3
+#define NVAMD_LINEAR_TILE_96X192 4
+#define NVAMD_LINEAR_TILE_256X128 5 /* two wave groups in turn */
+#define NVAMD_LINEAR_SMALL_M 6      /* weights streamed into registers, at most 256 tokens */
+#define NVAMD_LINEAR_FEW_TOKENS 7   /* at most 32 tokens, no barriers */
+#define NVAMD_LINEAR_FEW_TOKENS_X 8 /* the same, which quantises its activations */
+int32_t nvamd_fp8_linear_kernel(int64_t M, int64_t N, int64_t K, int32_t quantised, int64_t* lds_bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -393,10 +393,10 @@ nvamd::Fp8GemmParams gemm_params(const void* xq, const void* x_scale, const void
 // The GEMM on quantised activations: the kernel its sizes call for.
 int32_t run_block_gemm(const char* fn, const nvamd::Fp8GemmParams& p, bool f16_out, void* workspace,
                        int64_t workspace_bytes, hipStream_t stream) {
-  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(p.M, p.N, p.Kc, device_cu_count(), false);
+  const int64_t lds_limit = device_lds_limit();
+  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(p.M, p.N, p.Kc, device_cu_count(), lds_limit, false);
   if (thin.mf > 0)
     return launch_status(nvamd::launch_fp8_thin_linear(p, thin, nullptr, 0, false, f16_out, stream), fn);
-  const int64_t lds_limit = device_lds_limit();
   const nvamd::SkinnyPlan plan = nvamd::fp8_skinny_plan(p.M, p.N, p.Kc, device_cu_count(), workspace_bytes, lds_limit);
   if (plan.cw > 0)
     return launch_status(nvamd::launch_fp8_skinny_gemm(p, plan, f16_out, static_cast<float*>(workspace), stream), fn);
@@ -427,9 +427,29 @@ int32_t nvamd_fp8_block_gemm(const void* xq, const void* x_scale, const void* we
                         out_dtype == NVAMD_DTYPE_F16, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+int32_t nvamd_fp8_linear_kernel(int64_t M, int64_t N, int64_t K, int32_t quantised, int64_t* lds_bytes) {
+  if (lds_bytes) *lds_bytes = 0;
+  if (M <= 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > 0x7fffffffll || K > 0x7fffffffll) return -1;
+  const int Kc = (int)(K / 128), cus = device_cu_count();
+  const int64_t lds_limit = device_lds_limit();
+  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(M, N, Kc, cus, lds_limit, quantised == 0);
+  if (thin.mf > 0) {
+    if (lds_bytes) *lds_bytes = thin.lds;
+    return thin.xi > 0 ? NVAMD_LINEAR_FEW_TOKENS_X : NVAMD_LINEAR_FEW_TOKENS;
+  }
+  const nvamd::SkinnyPlan plan = nvamd::fp8_skinny_plan(M, N, Kc, cus, INT64_MAX, lds_limit);
+  if (plan.cw > 0) {
+    if (lds_bytes) *lds_bytes = nvamd::fp8_skinny_lds_bytes(plan);
+    return NVAMD_LINEAR_SMALL_M;
+  }
+  const int config = nvamd::fp8_gemm_pick_config(M, N, Kc, cus, lds_limit);
+  if (config >= 0 && lds_bytes) *lds_bytes = nvamd::fp8_gemm_lds_bytes(config, Kc);
+  return config;
+}
+
 int64_t nvamd_fp8_block_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > 0x7fffffffll || K > 0x7fffffffll) return 0;
-  if (nvamd::fp8_thin_plan(M, N, (int)(K / 128), device_cu_count(), true).xi > 0) return 0;
+  if (nvamd::fp8_thin_plan(M, N, (int)(K / 128), device_cu_count(), device_lds_limit(), true).xi > 0) return 0;
   return act_bytes(M, K) + nvamd_fp8_block_gemm_workspace_bytes(M, N, K);
 }
 
@@ -446,7 +466,7 @@ int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype
   const bool f16 = x_dtype == NVAMD_DTYPE_F16;
   nvamd::Fp8GemmParams p =
       gemm_params(nullptr, nullptr, weight, weight_stride0, weight_scale, out, out_stride0, M, N, K);
-  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(M, N, p.Kc, device_cu_count(), true);
+  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(M, N, p.Kc, device_cu_count(), device_lds_limit(), true);
   if (thin.xi > 0)
     return launch_status(nvamd::launch_fp8_thin_linear(p, thin, x, x_stride0, f16, f16, (hipStream_t)stream), fn);
   const int64_t act = act_bytes(M, K);

@@ -207,17 +207,17 @@ __global__ __launch_bounds__(64 * kThinMaxWaves) void thin_linear_kernel(Fp8Gemm
 }
 
 template <int MF, int XI, bool F16_IN>
-hipError_t launch_thin(const Fp8GemmParams& p, const void* x, int64_t x_stride, int nw, bool f16_out,
+hipError_t launch_thin(const Fp8GemmParams& p, const ThinPlan& pl, const void* x, int64_t x_stride, bool f16_out,
                        hipStream_t stream) {
   auto kern = thin_linear_kernel<MF, XI, F16_IN>;
-  const int lds = thin_lds_bytes(nw, (int)p.M, XI);
+  const int lds = pl.lds;
   static std::atomic<int> lds_set{0};  // largest dynamic LDS size granted so far
   if (lds > lds_set.load(std::memory_order_relaxed)) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
     lds_set.store(lds, std::memory_order_relaxed);
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)(p.N / 16)), dim3((unsigned)(64 * nw)), (size_t)lds, stream, p,
+  hipLaunchKernelGGL(kern, dim3((unsigned)(p.N / 16)), dim3((unsigned)(64 * pl.nw)), (size_t)lds, stream, p,
                      (const uint16_t*)x, x_stride, f16_out ? 1 : 0);
   return hipGetLastError();
 }
@@ -236,37 +236,42 @@ hipError_t launch_thin(const Fp8GemmParams& p, const void* x, int64_t x_stride, 
 // Its own quantisation repeats per workgroup and pays for one or two tokens
 // (6,144 x 4,096, M = 2: 8.0 against 10.3; M = 4: 12.6 against 10.3), up to
 // four when every workgroup has a CU (4,096 x 4,096, M = 4: 7.6 against 10.3).
-ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, bool raw_x) {
+ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit, bool raw_x) {
   ThinPlan pl;
   if (M < 1 || M > kThinMaxM || N % 128 != 0 || Kc < 1 || M * Kc > (1 << 11) || M * N > 600000) return pl;
   // Waves: the chunks in equal rounds, of at most four waves (two workgroups a
   // CU) or, when a CU has one workgroup at most, eight (12,288 columns: six
   // waves twice 11.4 us, four waves three times 13.4; 25,600 columns, 320
-  // workgroups: four waves 27.3, five 33.2 with one workgroup a CU).
+  // workgroups: four waves 27.3, five 33.2 with one workgroup a CU), and of as
+  // many as fit the LDS (the slices of four quantised tokens leave room for
+  // seven).
   const int chunks = (Kc + kThinKb - 1) / kThinKb;
   const bool one_wg = N / 16 <= cus;
-  const int most = one_wg ? kThinMaxWaves : 4;
+  const int xi = !raw_x || M > (one_wg ? 4 : 2) ? 0 : M <= 1 ? 2 : M <= 2 ? 4 : 8;
+  const int most = (int)std::min<int64_t>(one_wg ? kThinMaxWaves : 4, lds_limit / thin_lds_bytes(1, (int)M, xi));
+  if (most < 1) return pl;
   const int rounds = (chunks + most - 1) / most;
   pl.nw = (chunks + rounds - 1) / rounds;
   pl.mf = M <= 16 ? 1 : 2;
-  pl.xi = !raw_x || M > (one_wg ? 4 : 2) ? 0 : M <= 1 ? 2 : M <= 2 ? 4 : 8;
+  pl.xi = xi;
+  pl.lds = thin_lds_bytes(pl.nw, (int)M, xi);
   return pl;
 }
 
 hipError_t launch_fp8_thin_linear(const Fp8GemmParams& p, const ThinPlan& pl, const void* x, int64_t x_stride,
                                   bool f16_in, bool f16_out, hipStream_t stream) {
   if (pl.mf == 0 || p.M < 1 || p.M > 16 * pl.mf || pl.nw < 1 || pl.nw > kThinMaxWaves || p.N % 16 != 0 ||
-      (pl.xi > 0 && p.M * kThinKb > 4 * pl.xi))
+      (pl.xi > 0 && p.M * kThinKb > 4 * pl.xi) || pl.lds < thin_lds_bytes(pl.nw, (int)p.M, pl.xi))
     return hipErrorInvalidValue;
   switch (pl.xi > 0 ? 16 * pl.xi + (f16_in ? 1 : 0) : pl.mf) {
-    case 1: return launch_thin<1, 0, false>(p, nullptr, 0, pl.nw, f16_out, stream);
-    case 2: return launch_thin<2, 0, false>(p, nullptr, 0, pl.nw, f16_out, stream);
-    case 32: return launch_thin<1, 2, false>(p, x, x_stride, pl.nw, f16_out, stream);
-    case 33: return launch_thin<1, 2, true>(p, x, x_stride, pl.nw, f16_out, stream);
-    case 64: return launch_thin<1, 4, false>(p, x, x_stride, pl.nw, f16_out, stream);
-    case 65: return launch_thin<1, 4, true>(p, x, x_stride, pl.nw, f16_out, stream);
-    case 128: return launch_thin<1, 8, false>(p, x, x_stride, pl.nw, f16_out, stream);
-    case 129: return launch_thin<1, 8, true>(p, x, x_stride, pl.nw, f16_out, stream);
+    case 1: return launch_thin<1, 0, false>(p, pl, nullptr, 0, f16_out, stream);
+    case 2: return launch_thin<2, 0, false>(p, pl, nullptr, 0, f16_out, stream);
+    case 32: return launch_thin<1, 2, false>(p, pl, x, x_stride, f16_out, stream);
+    case 33: return launch_thin<1, 2, true>(p, pl, x, x_stride, f16_out, stream);
+    case 64: return launch_thin<1, 4, false>(p, pl, x, x_stride, f16_out, stream);
+    case 65: return launch_thin<1, 4, true>(p, pl, x, x_stride, f16_out, stream);
+    case 128: return launch_thin<1, 8, false>(p, pl, x, x_stride, f16_out, stream);
+    case 129: return launch_thin<1, 8, true>(p, pl, x, x_stride, f16_out, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -170,18 +170,19 @@ struct SkinnyPlan {
 };
 SkinnyPlan fp8_skinny_plan(int64_t M, int64_t N, int Kc, int cus, int64_t workspace_bytes, int64_t lds_limit);
 int64_t fp8_skinny_workspace_bytes(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit);
+int64_t fp8_skinny_lds_bytes(const SkinnyPlan& plan);
 hipError_t launch_fp8_skinny_gemm(const Fp8GemmParams& p, const SkinnyPlan& plan, bool f16_out, float* part,
                                   hipStream_t stream);
 
 // Linear for at most kThinMaxM tokens in one launch (fp8_thin_linear.hip): nw
 // waves per workgroup, mf 16-token fragments; xi > 0: the kernel quantises x
 // itself (xi passes of four groups per wave and chunk), else it reads the
-// quantised activations.  mf == 0: no plan.
+// quantised activations; lds bytes of LDS per workgroup.  mf == 0: no plan.
 constexpr int64_t kThinMaxM = 32;
 struct ThinPlan {
-  int nw = 0, mf = 0, xi = 0;
+  int nw = 0, mf = 0, xi = 0, lds = 0;
 };
-ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, bool raw_x);
+ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit, bool raw_x);
 hipError_t launch_fp8_thin_linear(const Fp8GemmParams& p, const ThinPlan& plan, const void* x, int64_t x_stride,
                                   bool f16_in, bool f16_out, hipStream_t stream);
 

@@ -58,6 +58,7 @@ SIGNATURES = {
     "nvamd_fp8_block_linear": (_i32, [_c_void_p, _i64, _i32, _c_void_p, _i64, _c_void_p, _c_void_p, _i64,
                                       _i64, _i64, _i64, _c_void_p, _i64, _c_void_p]),
     "nvamd_fp8_block_linear_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "nvamd_fp8_linear_kernel": (_i32, [_i64, _i64, _i64, _i32, ctypes.POINTER(_i64)]),
     "nvamd_prefill_workspace_bytes": (_i64, [_i64, _i32, _i32, _i32, _i64, _i32, _i32, _i32]),
     "nvamd_fp8_prefill_attention": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                            _c_void_p, _c_void_p, _i64, _i32, _i32, _i32, _i32,

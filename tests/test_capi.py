@@ -95,3 +95,21 @@ def test_fp8_linear_rejects_bad_shapes_without_gpu():
     assert b"null workspace" in lib.nvamd_last_error()
     assert lib.nvamd_fp8_block_gemm_workspace_bytes(0, 256, 256) == 0
     assert lib.nvamd_fp8_block_gemm_workspace_bytes(4, 200, 256) == 0
+
+
+@pytest.mark.parametrize("quantised", [0, 1])
+def test_fp8_linear_plans_fit_the_lds_without_gpu(quantised):
+    """Every size has a kernel, and its workgroups ask for no more LDS than a
+    gfx950 workgroup can have: few tokens over all K (four tokens of K 7,296 to
+    8,192 with eight waves that quantise would ask for 165,376 bytes), each
+    kernel at its largest sizes."""
+    lib = _native.load()
+    lds = ctypes.c_int64()
+    for M in [*range(1, 34), 64, 129, 192, 193, 256, 257, 1888, 8192]:
+        for N in (128, 1280, 4096, 4224, 24576, 51200):
+            for K in range(128, 32768 + 128, 128 if M <= 5 else 1920):
+                kernel = lib.nvamd_fp8_linear_kernel(M, N, K, quantised, ctypes.byref(lds))
+                assert 0 <= kernel <= 8, (M, N, K)
+                assert 0 < lds.value <= 160 * 1024, (M, N, K, kernel, lds.value)
+                if quantised == 0:
+                    assert (lib.nvamd_fp8_block_linear_workspace_bytes(M, N, K) == 0) == (kernel == 8), (M, N, K)

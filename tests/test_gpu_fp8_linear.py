@@ -306,13 +306,15 @@ def test_skinny_gemm_matches_oracle(M, N, K, out_dtype):
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(128, 128), (256, 1024), (384, 1152), (1024, 3072), (4224, 640), (4352, 2176),
-                                 (512, 12288), (4224, 5248)])
+                                 (512, 12288), (4224, 5248), (256, 4096), (128, 5120), (4224, 4096), (256, 7168),
+                                 (512, 8192), (4096, 8192), (256, 16384)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_tokens(M, N, K, dtype):
     """Calls of at most 32 tokens: one K block to several chunks of eight per
-    wave with a short last one, one to eight waves, one workgroup a CU or more,
-    activations quantised in the kernel (up to 2 or 4 tokens) and read
-    quantised, strided activation rows.  Random codes against the oracle; the
+    wave with a short last one, one to eight waves (six and four where the
+    slices of four quantised tokens leave no room for eight), one workgroup a
+    CU or more, activations quantised in the kernel (up to 2 or 4 tokens) and
+    read quantised, strided activation rows.  Random codes against the oracle; the
     same call on activations quantised beforehand adds the same products in
     the same order, so it gives the same bits."""
     g = torch.Generator().manual_seed(M + 3 * N + K)
