@@ -242,19 +242,22 @@ ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit,
   // Waves: the chunks in equal rounds, of at most four waves (two workgroups a
   // CU) or, when a CU has one workgroup at most, eight (12,288 columns: six
   // waves twice 11.4 us, four waves three times 13.4; 25,600 columns, 320
-  // workgroups: four waves 27.3, five 33.2 with one workgroup a CU), and of as
-  // many as fit the LDS (the slices of four quantised tokens leave room for
-  // seven).
+  // workgroups: four waves 27.3, five 33.2 with one workgroup a CU).
   const int chunks = (Kc + kThinKb - 1) / kThinKb;
   const bool one_wg = N / 16 <= cus;
-  const int xi = !raw_x || M > (one_wg ? 4 : 2) ? 0 : M <= 1 ? 2 : M <= 2 ? 4 : 8;
-  const int most = (int)std::min<int64_t>(one_wg ? kThinMaxWaves : 4, lds_limit / thin_lds_bytes(1, (int)M, xi));
-  if (most < 1) return pl;
+  const int most = one_wg ? kThinMaxWaves : 4;
   const int rounds = (chunks + most - 1) / most;
-  pl.nw = (chunks + rounds - 1) / rounds;
+  const int nw = (chunks + rounds - 1) / rounds;
+  // The waves do not depend on who quantises, so neither do the sums: where
+  // the slices do not fit beside the chunks (four tokens and eight waves), the
+  // activations are quantised before.
+  int xi = !raw_x || M > (one_wg ? 4 : 2) ? 0 : M <= 1 ? 2 : M <= 2 ? 4 : 8;
+  if (thin_lds_bytes(nw, (int)M, xi) > lds_limit) xi = 0;
+  if (thin_lds_bytes(nw, (int)M, xi) > lds_limit) return pl;
+  pl.nw = nw;
   pl.mf = M <= 16 ? 1 : 2;
   pl.xi = xi;
-  pl.lds = thin_lds_bytes(pl.nw, (int)M, xi);
+  pl.lds = thin_lds_bytes(nw, (int)M, xi);
   return pl;
 }
 

@@ -311,10 +311,10 @@ def test_skinny_gemm_matches_oracle(M, N, K, out_dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_tokens(M, N, K, dtype):
     """Calls of at most 32 tokens: one K block to several chunks of eight per
-    wave with a short last one, one to eight waves (six and four where the
-    slices of four quantised tokens leave no room for eight), one workgroup a
-    CU or more, activations quantised in the kernel (up to 2 or 4 tokens) and
-    read quantised, strided activation rows.  Random codes against the oracle; the
+    wave with a short last one, one to eight waves, one workgroup a CU or more,
+    activations quantised in the kernel (up to 2 or 4 tokens; three with eight
+    waves, which with four would need more LDS than there is) and read
+    quantised, strided activation rows.  Random codes against the oracle; the
     same call on activations quantised beforehand adds the same products in
     the same order, so it gives the same bits."""
     g = torch.Generator().manual_seed(M + 3 * N + K)
