@@ -354,8 +354,10 @@ __global__ __launch_bounds__(512) void swap_gemm_kernel(Fp8GemmParams p) {
   const int Kc = p.Kc;
   const int rows_x = (int)min((int64_t)T::BM, p.M - m0);  // valid token rows of the tile
 
-  // descriptors as in the tile kernel
-  const u32x4 rw = rsrc_words(p.w + (int64_t)n0 * p.w_stride, (uint32_t)((int64_t)T::BN * p.w_stride));
+  // descriptors as in the tile kernel, but that of the weights ends with the
+  // last row's K bytes: stages past the last are issued here, and rows further
+  // apart than K bytes (a column slice) need not have bytes after them
+  const u32x4 rw = rsrc_words(p.w + (int64_t)n0 * p.w_stride, (uint32_t)((int64_t)(T::BN - 1) * p.w_stride + p.K));
   const u32x4 rx = rsrc_words(p.xq + m0 * p.x_row, x_bytes(p, rows_x));
   const u32x4 rsx = rsrc_words(p.x_scale + m0 * p.sx_row, sx_bytes(p, rows_x));
   const int64_t sw_first = (int64_t)(n0 / kFp8Block) * Kc;

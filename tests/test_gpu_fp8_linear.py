@@ -391,3 +391,31 @@ def test_group_swap_tiles(M, N, K):
         absum += torch.matmul(xb.abs(), wb.abs()) * s
     bad = (got - acc.double()).abs() > 2.0 ** -7 * acc.double().abs() + ABS_TOL * absum.double()
     assert not bad.any(), f"{int(bad.sum())} outputs off, first at {bad.nonzero()[0].tolist()}"
+
+
+@pytest.mark.parametrize("kernel,M,N,K", [(0, 3851, 4096, 384), (5, 1793, 4096, 1152), (1, 1001, 2048, 512),
+                                          (4, 100, 24576, 640), (6, 77, 2048, 2176), (7, 9, 512, 1152)])
+def test_weights_in_the_last_columns_of_a_wider_matrix(kernel, M, N, K):
+    """Weights that are the last K columns of a matrix with longer rows: the
+    last row ends with the matrix, so no kernel may read past its K bytes (the
+    matrix is the tail of one allocation).  Same bits as on contiguous
+    weights."""
+    announce(f"fp8 linear: GEMM {M} x {N} x {K}, weights in a wider matrix's last columns")
+    lib = _native.load()
+    assert lib.nvamd_fp8_linear_kernel(M, N, K, 1, None) == kernel
+    g = torch.Generator(device="cuda").manual_seed(K)
+    wide = torch.randint(0, 120, (N, K + 256), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    xq = torch.randint(0, 120, (M, K), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    xs = (torch.rand(M, K // 128, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    ws = (torch.rand(N // 128, K // 128, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    need = lib.nvamd_fp8_block_gemm_workspace_bytes(M, N, K)
+    work = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    outs = []
+    for w in (wide[:, 256:], wide[:, 256:].contiguous()):
+        out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        _native.check(lib.nvamd_fp8_block_gemm(xq.data_ptr(), xs.data_ptr(), w.data_ptr(), w.stride(0), ws.data_ptr(),
+                                               out.data_ptr(), N, 0, M, N, K, work.data_ptr() if need else None, need,
+                                               torch.cuda.current_stream().cuda_stream), "fp8_block_gemm")
+        outs.append(out.view(torch.int16))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
