@@ -461,8 +461,8 @@ int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype
                                workspace, workspace_bytes))
     return e;
   if (x_stride0 < K) return fail(NVAMD_ERR_INVALID_ARGUMENT, "%s: x row stride is shorter than a row", fn);
+  if (M == 0) return ok();  // no rows: any stride
   if (x_stride0 % 8 != 0) return fail(NVAMD_ERR_UNSUPPORTED, "%s: x row stride must be a multiple of 8 elements", fn);
-  if (M == 0) return ok();
   const bool f16 = x_dtype == NVAMD_DTYPE_F16;
   nvamd::Fp8GemmParams p =
       gemm_params(nullptr, nullptr, weight, weight_stride0, weight_scale, out, out_stride0, M, N, K);

@@ -113,3 +113,20 @@ def test_fp8_linear_plans_fit_the_lds_without_gpu(quantised):
                 assert 0 < lds.value <= 160 * 1024, (M, N, K, kernel, lds.value)
                 if quantised == 0:
                     assert (lib.nvamd_fp8_block_linear_workspace_bytes(M, N, K) == 0) == (kernel == 8), (M, N, K)
+
+
+def test_fp8_block_linear_checks_without_gpu():
+    """The checks of the whole layer are those of its two steps: an empty batch
+    (any row stride, null pointers) is accepted, a row stride that is shorter
+    than a row or, with rows, not a multiple of 8 elements is not."""
+    lib = _native.load()
+
+    def call(M, x_stride, x=None):
+        return lib.nvamd_fp8_block_linear(x, x_stride, 0, x, 128, x, x, 256, M, 256, 128, None, 0, None)
+
+    for stride in (128, 130, 132):
+        assert call(0, stride) == 0
+        assert lib.nvamd_fp8_act_quant(None, stride, 0, None, None, 0, 128, None) == 0
+    assert call(0, 100) == 1 and call(4, 100) == 1
+    assert call(4, 128) == 1 and b"null pointer" in lib.nvamd_last_error()
+    assert call(4, 132, x=0x1000) == 2 and b"row stride" in lib.nvamd_last_error()
