@@ -115,7 +115,10 @@ __global__ __launch_bounds__(64 * kThinMaxWaves) void thin_linear_kernel(Fp8Gemm
   for (int c = wave; c < chunks; c += nw) {
     const int kc0 = c * kThinKb;
     // activations first (loads complete in order), then the weights
-    const uint32_t sw_bits = sw_row[min(kc0 + (lane & (kThinKb - 1)), Kc - 1)];  // lane kb: scale of block kc0 + kb
+    // lane kb: scale of block kc0 + kb; blocks past K count as zero (not the
+    // last block's scale, which may be infinite: 0 * inf is NaN)
+    const int sw_kc = kc0 + (lane & (kThinKb - 1));
+    const uint32_t sw_bits = sw_kc < Kc ? (uint32_t)sw_row[sw_kc] : 0u;
     if constexpr (XI > 0) {
 #pragma unroll
       for (int i = 0; i < XI; ++i) {  // group 4 i + q: token (4 i + q) / 8, K block kc0 + (4 i + q) % 8

@@ -419,3 +419,23 @@ def test_weights_in_the_last_columns_of_a_wider_matrix(kernel, M, N, K):
         outs.append(out.view(torch.int16))
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 256, 1152), (2, 4352, 1152), (4, 256, 1664), (9, 256, 1152), (20, 512, 128),
+                                   (40, 256, 2176)])
+def test_infinite_weight_scale_in_the_last_block(M, N, K):
+    """A weight scale of +inf in the last K block (K not a multiple of the
+    chunks that kernels work in): the block's features are infinite with the
+    sign of the block's sum, the others finite."""
+    announce(f"fp8 linear: infinite scale in the last block, {M} x {N} x {K}")
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (torch.rand(M, K, generator=g) + 0.5).to(torch.bfloat16)
+    w = (torch.rand(N, K, generator=g) + 0.5).to(torch.float8_e4m3fn)
+    w[5] = -w[5].float()
+    w_scale = torch.full((N // 128, K // 128), 0.01, dtype=torch.bfloat16)
+    w_scale[0, -1] = float("inf")
+    got = fp8_block_linear(x.cuda(), w.cuda(), w_scale.cuda()).float().cpu()
+    want = torch.full((M, 128), float("inf"))
+    want[:, 5] = -float("inf")
+    assert torch.equal(got[:, :128], want), got[:, :8]
+    assert torch.isfinite(got[:, 128:]).all()
