@@ -697,6 +697,7 @@ int32_t decode_attention(const char* fn, void* out, const void* q, const void* k
     p.max_parts = 1;
     p.sk_heads = stream_k_heads(num_kv_heads, false);
     p.sk_wgs = stream_k_wgs(ncb, p.sk_heads, G, false);
+    p.sk_cus = device_cu_count();
     p.sk_cols = G;
     p.sk_prefix = static_cast<int32_t*>(workspace);
     p.sk_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + stream_k_prefix_bytes(batch));
@@ -837,6 +838,7 @@ int32_t nvamd_fp8_prefill_attention(void* out, const void* q, const void* k, con
     mp.max_parts = 1;
     mp.sk_heads = stream_k_heads(num_kv_heads, true);
     mp.sk_wgs = stream_k_wgs(ncb, mp.sk_heads, G, true);
+    mp.sk_cus = device_cu_count();
     mp.sk_cols = short_cols(G, max_seqlen_q);
     mp.sk_prefix = static_cast<int32_t*>(workspace);
     mp.sk_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + stream_k_prefix_bytes(num_seqs));

@@ -32,6 +32,7 @@ struct MqParams {
   float* sk_part;               // [sk_wgs, 2, sk_heads, sk_cols, kSkSlotFloats] partials (see kSkSlotFloats)
   int32_t* sk_prefix;           // [num_seqs + 1] stages per kv-head group before each sequence
   int sk_wgs;                   // persistent workgroups
+  int sk_cus;                   // CUs of the device
   int sk_heads;                 // kv heads per workgroup (4 or 8; one wave each)
   int sk_cols;                  // query columns per kv head: G (decode) or G * mq_max_q (varlen)
 };

@@ -91,35 +91,50 @@ __host__ __device__ __forceinline__ int merge_slices(const MqParams& p, int n_wa
 
 // ---- balanced (stream-K) kernel: merge of a pair cut across workgroups ----
 
-// Stream-K ranges of the balanced decode kernel.  Workgroup w gets a share
-// of the T stages proportional to its weight: a for even w, kSkPairWeight - a
-// for odd w.  Workgroups are dealt to the 8 XCDs round-robin, so even
-// workgroups run on even-numbered XCDs; on MI355X those stream this kernel's
-// KV bytes 5-10% faster than the odd-numbered ones when every CU is loading
-// at full rate (per-workgroup wall-clock timestamps, on several boxes), and
-// equal shares then leave the even XCDs idle at the end.  Decode runs at
-// that rate and takes a = kSkEvenWeight; the short-query rows of a varlen
-// call do not, and take equal shares.  The split is fixed, so results do
-// not depend on timing.  With C(w) = the weight of workgroups 0 .. w-1,
-// workgroup w owns stages [T C(w) / C(W), T C(w+1) / C(W)).
-constexpr int kSkPairWeight = 64, kSkEvenWeight = 33;
-
-__device__ __forceinline__ int sk_even_weight(const MqParams& p) {
-  return p.cu_q == nullptr ? kSkEvenWeight : kSkPairWeight / 2;
+// Workgroups that take stages, of a call with T stages: one stage each while
+// there are workgroups (T of them then share nothing but the merge), up to
+// one workgroup per CU; the rest of the grid (kernels of which a CU holds two
+// or three) from four stages each on.  A pair is cut into at most 64 ranges,
+// what the waves of the wide merge add in one round trip, unless those would
+// get more than four stages each.  us per call by workgroups (GPU time, 8 kv
+// heads, 32 query heads unless said otherwise; best of each):
+//   1 x 777 tokens (49 stages)        49: 11.7, 24: 12.6
+//   1 x 2,048 (128)                   128: 13.4, 64: 12.8, 32: 14.0
+//   1 x 4,096 (256)                   256: 16.3, 128: 14.4, 64: 14.5
+//   1 x 8,192 (512)                   256: 17.2, 128: 16.1, 64: 17.9
+//   64 x 16 (64)                      64: 9.7, 32: 13.2
+//   64 x 160 (640)                    256: 13.5, 160: 15.9, 128: 14.5
+//   32 of 1 to 320 (284)              256: 14.1, 128: 15.5
+//   4 / 4 heads, 4 x 4,096 (1,024)    768: 16.0, 512: 14.6, 256: 13.2
+//   4 x 5 rows on 777 (392)           384: 17.5, 256: 15.3, 128: 14.5
+// W <= T, so no range is empty (sk_even_weight) and every workgroup between a
+// cut pair's first and last owner left a partial.
+constexpr int kSkMaxRanges = 64;
+__device__ __forceinline__ int sk_active_wgs(const MqParams& p, int NHG, int64_t T) {
+  int W = p.sk_cus;
+  while (W < p.sk_wgs && T >= 4 * (int64_t)W + p.sk_cus) W += p.sk_cus;
+  W = min(W, p.sk_wgs);
+  if (T < 4 * (int64_t)p.sk_cus) W = min(min(W, (int)T), max(kSkMaxRanges * p.num_seqs * NHG, (int)T / 4));
+  return max(W, 1);
 }
 
-// Workgroups that take stages.  Every one of them gets two stages or more, so
-// no range is empty (a weighted share is at least 31/32 of the mean) and
-// every workgroup between a cut pair's first and last owner left a partial.
-// A call too small to give the whole grid four stages each uses half of the
-// grid at most: what such a call costs is the chain load -> partial -> merge,
-// and a stage more per workgroup costs it less than twice the contributors
-// (one sequence on 8 kv heads, us per call, at least 1 / 2 / 4 stages each:
-// 64 tokens 10.2 / 11.1 / 11.9, 777 tokens 12.4 / 12.4 / 14.0, 2,048 tokens
-// 13.4 / 13.3 / 14.5, 8,192 tokens 17.9 / 17.8 / 16.6).
-__device__ __forceinline__ int sk_active_wgs(const MqParams& p, int64_t T) {
-  const int64_t n = max(min(T / 2, (int64_t)p.sk_wgs / 2), T / 4);
-  return (int)max((int64_t)1, min((int64_t)p.sk_wgs, n));
+// Stream-K ranges of the balanced decode kernel.  Workgroup w of W gets a
+// share of the T stages proportional to its weight: a for even w,
+// kSkPairWeight - a for odd w.  Workgroups are dealt to the 8 XCDs
+// round-robin, so even workgroups run on even-numbered XCDs; on MI355X those
+// stream this kernel's KV bytes 5-10% faster than the odd-numbered ones when
+// every CU is loading at full rate (per-workgroup wall-clock timestamps, on
+// several boxes), and equal shares then leave the even XCDs idle at the end.
+// Decode on the whole grid runs at that rate and takes a = kSkEvenWeight
+// (from two stages each on: 31 / 32 of them is still more than one); smaller
+// calls and the short-query rows of a varlen call do not, and take equal
+// shares.  The split is fixed, so results do not depend on timing.  With
+// C(w) = the weight of workgroups 0 .. w-1, workgroup w owns stages
+// [T C(w) / C(W), T C(w+1) / C(W)).
+constexpr int kSkPairWeight = 64, kSkEvenWeight = 33;
+
+__device__ __forceinline__ int sk_even_weight(const MqParams& p, int64_t T, int W) {
+  return p.cu_q == nullptr && W == p.sk_wgs && T >= 2 * (int64_t)W ? kSkEvenWeight : kSkPairWeight / 2;
 }
 
 // C(w) in the integer type U (uint32_t when T * C(W) + T < 2^32, see
@@ -189,13 +204,13 @@ __device__ __forceinline__ void sk_merge_one(const MqParams& p, int b, int idx, 
     return;
   }
   const int64_t T = (int64_t)NHG * p.sk_prefix[p.num_seqs];
-  const int W = sk_active_wgs(p, T);
+  const int W = sk_active_wgs(p, NHG, T);
   const int64_t P = (int64_t)NHG * pre_b + (int64_t)hg * n;
   // owners of the pair's first and last stages, and wf's slot (below); in
   // 32-bit arithmetic when T * (W + 1) < 2^32 (every product below is then
   // below 2^32), since a 64-bit division is a long instruction sequence and
   // this pass runs one per wave
-  const int a = sk_even_weight(p);
+  const int a = sk_even_weight(p, T, W);
   int wf, wl, slot_f;
   if (sk_fits32(T, W, a)) sk_pair_owners<uint32_t>((uint32_t)P, (uint32_t)n, (uint32_t)T, (uint32_t)W, (uint32_t)a, wf, wl, slot_f);
   else sk_pair_owners<uint64_t>((uint64_t)P, (uint64_t)n, (uint64_t)T, (uint64_t)W, (uint64_t)a, wf, wl, slot_f);
@@ -341,9 +356,9 @@ __device__ __forceinline__ void sk_merge_cols(const MqParams& p, int b, int kvh,
     return;
   }
   const int64_t T = (int64_t)NHG * p.sk_prefix[p.num_seqs];
-  const int W = sk_active_wgs(p, T);
+  const int W = sk_active_wgs(p, NHG, T);
   const int64_t P = (int64_t)NHG * pre_b + (int64_t)hg * n;
-  const int a = sk_even_weight(p);
+  const int a = sk_even_weight(p, T, W);
   int wf, wl, slot_f;
   if (sk_fits32(T, W, a)) sk_pair_owners<uint32_t>((uint32_t)P, (uint32_t)n, (uint32_t)T, (uint32_t)W, (uint32_t)a, wf, wl, slot_f);
   else sk_pair_owners<uint64_t>((uint64_t)P, (uint64_t)n, (uint64_t)T, (uint64_t)W, (uint64_t)a, wf, wl, slot_f);

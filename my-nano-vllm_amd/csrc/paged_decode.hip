@@ -712,14 +712,16 @@ __global__ __launch_bounds__(64 * HG) void decode_sk_kernel(MqParams p, PrefillP
     __syncthreads();
   }
   const int64_t T = (int64_t)NHG * carry;
-  if (w == 0)
-    for (int b = tid; b <= B; b += kThreads) p.sk_prefix[b] = pre[b];
   // this workgroup's share of the stages (sk_range_start)
-  const int W = sk_active_wgs(p, T);
+  const int W = sk_active_wgs(p, NHG, T);
+  // the prefix, for the merge: by a workgroup without stages if there is one
+  // (its loads would wait for the stores)
+  if (w == (W < p.sk_wgs ? W : 0))
+    for (int b = tid; b <= B; b += kThreads) p.sk_prefix[b] = pre[b];
   if (w >= W) return;
   int64_t start, end;
   {
-    const int a = sk_even_weight(p);
+    const int a = sk_even_weight(p, T, W);
     if (sk_fits32(T, W, a)) {
       start = sk_range_start<uint32_t>(w, (uint32_t)T, W, a);
       end = sk_range_start<uint32_t>(w + 1, (uint32_t)T, W, a);
@@ -1123,7 +1125,7 @@ hipError_t launch_decode_sk(const MqParams& p, int ncb, bool merge, const Prefil
   const bool heads_at_once = !varlen && p.G <= 4;
   const int groups = (p.G * p.mq_max_q + 3) / 4;  // of four query columns
   const int64_t wide_wgs = (int64_t)p.num_seqs * p.Hkv * groups;
-  if (wide_wgs <= kSkWideMaxWgs && (int64_t)p.num_seqs * (p.Hkv / hg) * (heads_at_once ? 8 : 16) <= p.sk_wgs)
+  if (wide_wgs <= kSkWideMaxWgs && (int64_t)p.num_seqs * (p.Hkv / hg) * (heads_at_once ? 8 : 16) < p.sk_wgs)
     hipLaunchKernelGGL(decode_sk_merge_wide_kernel, dim3((unsigned)wide_wgs), dim3(64 * kSkWideWaves), 0, stream, p,
                        groups);
   else if (heads_at_once)

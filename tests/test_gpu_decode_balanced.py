@@ -163,12 +163,14 @@ def test_balanced_decode_garbage_and_reused_workspace():
 
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (64, 8), (8, 4), (24, 8)])
 @pytest.mark.parametrize("ctx", [[1], [16], [17], [33], [49], [777], [4079], [4096], [8191], [16400], [40000],
-                                 [5, 0, 700], [1, 9000, 64], [300] * 5], ids=str)
+                                 [5, 0, 700], [1, 9000, 64], [300] * 5, [2048, 2100], [16] * 40, [64] * 130,
+                                 [160, 33, 1] * 25, [90] * 256],
+                         ids=lambda c: f"{len(c)}x{c[0]}" if len(c) > 5 else str(c))
 def test_balanced_decode_few_pairs(hq, hkv, ctx):
-    """Few pairs: from one stage on one workgroup, over calls that use half of
-    the grid (two to four stages each), to pairs cut into every range, whose
-    partials several waves combine; after a call that left the workspace's
-    partials full of another call's values."""
+    """Small calls: from one stage on one workgroup, over one stage each on as
+    many workgroups as there are stages and one workgroup per CU, to two per CU
+    and to pairs cut into every range, whose partials several waves combine; in
+    a workspace full of NaN."""
     seqs = [W.SeqSpec(lq=1, cached=max(c, 1) - 1) for c in ctx]
     wl = W.make_workload(f"few_{hq}_{hkv}_{ctx}", hq, hkv, seqs, seed=sum(ctx) + hq)
     announce(f"balanced decode: few pairs {hq}/{hkv} ctx={ctx}")
