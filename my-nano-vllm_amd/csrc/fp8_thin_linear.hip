@@ -115,10 +115,7 @@ __global__ __launch_bounds__(64 * kThinMaxWaves) void thin_linear_kernel(Fp8Gemm
   for (int c = wave; c < chunks; c += nw) {
     const int kc0 = c * kThinKb;
     // activations first (loads complete in order), then the weights
-    // lane kb: scale of block kc0 + kb; blocks past K count as zero (not the
-    // last block's scale, which may be infinite: 0 * inf is NaN)
-    const int sw_kc = kc0 + (lane & (kThinKb - 1));
-    const uint32_t sw_bits = sw_kc < Kc ? (uint32_t)sw_row[sw_kc] : 0u;
+    const uint32_t sw_bits = sw_row[min(kc0 + (lane & (kThinKb - 1)), Kc - 1)];  // lane kb: scale of block kc0 + kb
     if constexpr (XI > 0) {
 #pragma unroll
       for (int i = 0; i < XI; ++i) {  // group 4 i + q: token (4 i + q) / 8, K block kc0 + (4 i + q) % 8
@@ -153,7 +150,9 @@ __global__ __launch_bounds__(64 * kThinMaxWaves) void thin_linear_kernel(Fp8Gemm
     wait_vmcnt<0>();
     // this wave's chunk and slice are in LDS; no other wave touches them
     asm volatile("" ::: "memory");
-    const float sw_lane = bf16_bits_to_f32(sw_bits);
+    // blocks past K count as zero, not with the last block's scale (it may be
+    // infinite, and 0 * inf is NaN)
+    const float sw_lane = kc0 + (lane & (kThinKb - 1)) < Kc ? bf16_bits_to_f32(sw_bits) : 0.f;
 #pragma unroll
     for (int kb = 0; kb < kThinKb; ++kb) {
       const float sw = readlane_f32(sw_lane, kb);
