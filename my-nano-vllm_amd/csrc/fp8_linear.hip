@@ -934,16 +934,20 @@ SkinnyPlan fp8_skinny_plan(int64_t M, int64_t N, int Kc, int cus, int64_t worksp
   SkinnyPlan best;
   if (M < 1 || M > kSkinnyMaxM || N % 128 != 0 || Kc < 1 || (int64_t)Kc * kFp8Block >= (1 << 24) || cus < 1)
     return best;
-  // A tile grid that covers the CUs keeps them busier (measured at 192
-  // tokens: gate/up, 576 tiles of 128 x 64, 41.8 us against 50 us here); the
-  // small-M kernel is for grids that would leave CUs idle (qkv 144 tiles:
-  // 27.3 -> 24.3 us; down 96 tiles: 63.7 -> 35.3 us, weights streamed from
-  // HBM).  Nor for short rows, where a K split has nothing to gain (us per
-  // call, tiles against this kernel: 256 tokens on 6,144 x 4,096 29.8 / 37.9,
-  // but 29.5 / 28.1 on 4,096 x 4,096 and 69 / 49 on 4,096 x 12,288; 64 tokens
-  // on 1,024 x 2,048 10.4 / 13.6, 192 tokens 14.9 / 14.3).
-  if ((N / 128) * ((M + 63) / 64) >= cus) return best;
-  if (M > 192 ? Kc < 64 && (N > 4096 || N * Kc * kFp8Block <= (4 << 20)) : M <= 128 && N * Kc * kFp8Block <= (4 << 20)) return best;
+  // Where the tile kernels are faster (GPU time of both sides on 41 shapes of K
+  // 128 to 32,768 and N 128 to 51,200; profiles/fp8_linear_kernels.md):
+  //  - their grid covers the CUs, with 64-feature tiles for 64 tokens too (us
+  //    per call, tiles / this kernel: 64 tokens on 24,576 x 4,096 34.2 / 40.1,
+  //    on 19,456 x 2,560 22.9 / 33.9; but on 10,240 x 5,120 32.4 / 28.3);
+  //  - short rows, where a K split has little to share out.  The tiles' time is
+  //    one K block after another whatever M is, this kernel's grows with M, so
+  //    the line moves up with it: 64 tokens on 1,024 x 2,048 10.6 / 10.4 (and a
+  //    launch fewer), on 1,024 x 3,072 13.7 / 10.9; 128 on 1,024 x 2,048 10.7 /
+  //    12.8, on 6,144 x 2,560 18.4 / 18.9, on 1,024 x 4,096 16.8 / 14.2; 192 on
+  //    5,120 x 3,200 22.1 / 29.1, on 1,024 x 4,096 17.5 / 15.9; 256 on 4,096 x
+  //    4,096 26.5 / 28.1, on 1,024 x 6,144 24.8 / 21.3.
+  if ((N / 128) * ((M + 63) / 64) >= cus || N / 64 >= cus) return best;
+  if (Kc <= (M <= 32 ? 5 : M <= 64 ? 16 : M <= 128 ? 20 : M <= 192 ? 25 : 40)) return best;
   const int mf = M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : M <= 128 ? 8 : M <= 192 ? 12 : 16;
   // Estimated time (us): a workgroup's K blocks are latency-bound, about
   // 0.40 + 0.19 CW us each at 192 tokens (less with fewer token fragments),
@@ -1011,16 +1015,28 @@ hipError_t launch_fp8_act_quant(const void* x, int64_t x_stride, bool f16_in, vo
 }
 
 // Estimated time (us) of a product on configuration 0, 1 or 5, from sweeps of
-// 300 to 4,096 tokens over seven Qwen3 projections: a CU takes one large tile
-// at a time, 1.75 (256 x 256) or 1.15 (256 x 128) us per K block with all CUs
-// busy and 1.3 or 0.95 with few, plus 3 to 5 us to fill and drain; 128 x 64
-// tiles share a CU, 0.4 us per K block each.
-static double gemm_estimate(int config, int64_t tiles, int Kc, int cus) {
-  const double x = (double)tiles / cus;
-  if (config == 1) return 1.0 + Kc * std::max(0.85, 0.15 + 0.40 * x);
-  const double full = config == 0 ? 1.75 : 1.15, few = config == 0 ? 1.3 : 0.95;
-  const double whole = std::floor(x), part = x - whole;
-  return (config == 0 ? 3.0 : 5.0) + Kc * (whole * full + (part > 0 ? few + (full - few) * part : 0.0));
+// 65 to 8,192 tokens over 40 shapes (profiles/fp8_linear_kernels.md; the pick
+// is within 0.3 % of the fastest in the mean).  A CU takes one large tile at a
+// time, 1.75 (256 x 256) or 1.15 (256 x 128) us per K block with all CUs busy
+// and 1.3 or 0.95 with few, and 6 or 5 us to fill and drain each (6,144 x 1,024
+// at 1,536 tokens: 30.2 on 256 x 256, 26.0 on 128 x 64); 128 x 64 tiles share a
+// CU, 0.4 us per K block each.  Rows of tiles that cover more than half of the
+// CUs run one after another and read weights beyond the L2 again each (51,200 x
+// 5,120 at 257 tokens: 193 us on 128 x 64, 149 on 256 x 256).
+static double gemm_estimate(int config, int64_t M, int64_t N, int Kc, int cus) {
+  const int64_t rows = (M + kGemmBM[config] - 1) / kGemmBM[config];
+  const double x = (double)(N / kGemmBN[config] * rows) / cus;
+  double t;
+  if (config == 1) {
+    t = 1.0 + 0.3 * x + Kc * std::max(0.85, 0.15 + 0.40 * x);
+  } else {
+    const double full = config == 0 ? 1.75 : 1.15, few = config == 0 ? 1.3 : 0.95;
+    const double whole = std::floor(x), part = x - whole;
+    t = 3.0 + (config == 0 ? 6.0 : 5.0) * std::ceil(x) + Kc * (whole * full + (part > 0 ? few + (full - few) * part : 0.0));
+  }
+  const double weights = (double)N * Kc * kFp8Block;
+  if (N / 128 > cus / 2 && weights > (32 << 20)) t = std::max(t, 3.0 + (double)rows * weights / 7.6e6);
+  return t;
 }
 
 int fp8_gemm_pick_config(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit) {
@@ -1039,7 +1055,7 @@ int fp8_gemm_pick_config(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limi
     double best_t = 0.0;
     for (int c : {1, 5, 0}) {
       if (!fits(c)) continue;
-      const double t = gemm_estimate(c, tiles(c), Kc, cus);
+      const double t = gemm_estimate(c, M, N, Kc, cus);
       if (best < 0 || t < best_t) {
         best = c;
         best_t = t;

@@ -226,18 +226,28 @@ hipError_t launch_thin(const Fp8GemmParams& p, const ThinPlan& pl, const void* x
 
 }  // namespace
 
-// Where the kernel is taken, from both sides measured (us per call, weights
-// from HBM, quantisation included; this kernel / the small-M or tile kernel of
-// fp8_linear.hip).  Every workgroup reads all the activations, so it loses its
-// lead with M K (their bytes per workgroup) and with M N (their reads in all):
-//   6,144 x 4,096:   M 1 7.6 / 16.1, 8 10.5 / 16.6, 16 12.1 / 17.0, 32 16.3 / 18.4
-//   24,576 x 4,096:  M 1 20.2 / 42.3, 16 28.4 / 45.1, 24 35.2 / 47.6, 32 40.2 / 35.6
-//   4,096 x 12,288:  M 1 11.5 / 20.3, 16 17.8 / 20.8, 24 21.4 / 21.7, 32 23.4 / 21.9
-//   5,120 x 25,600:  M 1 27.4 / 40.0, 8 37.5 / 40.6, 12 41.7 / 40.8, 16 45.6 / 41.0
-//   51,200 x 5,120:  M 1 43.5 / 53.8, 8 48.8 / 55.5, 12 54.2 / 55.9, 16 60.3 / 57.5
+// Where the kernel is taken, from both sides measured (us per call, GPU time,
+// weights from HBM, quantisation included; this kernel / the fastest of
+// fp8_linear.hip; more in profiles/fp8_linear_kernels.md).  Every workgroup
+// reads all the activations, so it loses its lead with M K (their bytes per
+// workgroup) and with M N (their reads in all):
+//   6,144 x 4,096:   M 1 7.7 / 16.5, 8 10.7 / 17.0, 16 12.3 / 17.4, 32 16.1 / 18.7
+//   24,576 x 4,096:  M 1 21.4 / 30.8, 16 29.8 / 31.6, 24 34.8 / 32.8, 32 38.9 / 33.3
+//   4,096 x 12,288:  M 1 13.1 / 20.9, 16 17.6 / 21.4, 24 20.6 / 22.1, 32 23.0 / 22.3
+//   5,120 x 25,600:  M 1 31.5 / 41.7, 8 40.1 / 42.1, 12 43.9 / 42.4, 16 47.6 / 42.4
+//   51,200 x 5,120:  M 1 47.6 / 56.3, 8 52.8 / 57.6, 12 56.8 / 57.8, 16 61.4 / 58.2
+// With two workgroups on a CU a second token fragment doubles what the four
+// waves do per chunk:
+//   5,120 x 8,192:   M 16 18.7 / 20.0, 24 23.2 / 20.6
+//   6,144 x 1,024:   M 16 6.4 / 6.8, 24 7.5 / 7.0 (one wave per workgroup)
+// Few workgroups leave CUs idle, which a K split would use: worth it only for
+// what one round of chunks holds.
+//   512 x 8,192:     M 1 6.3 / 10.0, 16 11.3 / 10.9, 32 14.9 / 11.1
+//   512 x 12,288:    M 1 8.7 / 11.1, 3 12.2 / 11.6, 16 13.8 / 11.9 (two rounds)
+//   256 x 32,768:    M 1 15.0 / 14.9, 3 22.4 / 15.1 (four rounds)
 // Its own quantisation repeats per workgroup and pays for one or two tokens
-// (6,144 x 4,096, M = 2: 8.0 against 10.3; M = 4: 12.6 against 10.3), up to
-// four when every workgroup has a CU (4,096 x 4,096, M = 4: 7.6 against 10.3).
+// (6,144 x 4,096, M = 2: 8.3 against 10.3; M = 4: 12.6 against 10.3), up to
+// four when every workgroup has a CU (4,096 x 4,096, M = 4: 7.9 against 10.3).
 ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit, bool raw_x) {
   ThinPlan pl;
   if (M < 1 || M > kThinMaxM || N % 128 != 0 || Kc < 1 || M * Kc > (1 << 11) || M * N > 600000) return pl;
@@ -250,6 +260,8 @@ ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit,
   const int most = one_wg ? kThinMaxWaves : 4;
   const int rounds = (chunks + most - 1) / most;
   const int nw = (chunks + rounds - 1) / rounds;
+  if (N / 16 <= cus / 2 && M * Kc * rounds * rounds > (1 << 10)) return pl;
+  if (!one_wg && M > 16 && (chunks == 1 || M * Kc > 1280)) return pl;
   // The waves do not depend on who quantises, so neither do the sums: where
   // the slices do not fit beside the chunks (four tokens and eight waves), the
   // activations are quantised before.

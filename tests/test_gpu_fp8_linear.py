@@ -20,9 +20,10 @@ kernels: the 256x256 and 256x128 tiles whose two wave groups take turns, the
 4-stage ring for 33 to 192 tokens with at least a CU's worth of 96-feature tiles
 (tiles straddle the 128-row weight blocks, so fragments take their own scales;
 K shorter than the ring), the small-M kernel for products of at most 256 tokens
-whose tile grid would leave CUs idle (K split over workgroups with fp32 partials
-added in split order when the workspace allows), and the kernel for at most 32
-tokens that streams the weights without barriers.
+whose tile grid would leave CUs idle and whose rows are long enough to share out
+(K split over workgroups with fp32 partials added in split order when the
+workspace allows), and the kernel for at most 32 tokens that streams the weights
+without barriers.
 """
 import numpy as np
 import pytest
@@ -144,15 +145,17 @@ def test_act_quant_unit_scale_all_patterns_and_strided_rows():
     assert np.array_equal(_bits(xs), xs_ref)
 
 
-# (M, N, K): tile chosen on 256 CUs -> 256x256: (4096, 4096, 256), and (4096, 4096, 640) with an odd
-# number of K blocks (a token row's scale then sits in either half of its x_scale dword);
-# 128x64: (1024, 2048, 256); 128x32: (1024, 1024, 128); 64x16: (300, 128, 256)
-TILE_SHAPES = [(4096, 4096, 256), (4096, 4096, 640), (1024, 2048, 256), (1024, 1024, 128), (300, 128, 256)]
+# (M, N, K): tile chosen on 256 CUs -> 256x256: (4096, 4096, 640) with an odd number of K blocks (a token
+# row's scale then sits in either half of its x_scale dword); 256x128: (249, 24576, 1408); 128x64: (1024, 2048,
+# 256), (4096, 4096, 256); 128x32: (1024, 1024, 128); 64x16: (300, 128, 256), (77, 2048, 1664), (130, 512, 3200)
+TILE_SHAPES = [(4096, 4096, 256), (4096, 4096, 640), (1024, 2048, 256), (1024, 1024, 128), (300, 128, 256),
+               (249, 24576, 1408)]
 # at most 256 tokens: the Qwen3-8B qkv and down products at 192 tokens take the small-M kernel (down with K
-# split over workgroups), gate/up the 96x192 ring tile; 256 tokens (16 token fragments), one token (K split),
-# ragged token counts and odd K block counts on the small-M kernel
+# split over workgroups), gate/up the 96x192 ring tile; 256 tokens (16 token fragments), ragged token counts and
+# odd K block counts on the small-M kernel; one token and 24 on the kernel for few tokens
 SKINNY_SHAPES = [(192, 6144, 4096), (192, 24576, 4096), (192, 4096, 12288), (256, 1024, 4096), (1, 4096, 4096),
-                 (24, 256, 512), (1, 128, 128), (77, 2048, 1664), (130, 512, 3200)]
+                 (24, 256, 512), (1, 128, 128), (77, 2048, 1664), (130, 512, 3200), (256, 1024, 6144),
+                 (77, 2048, 2688), (130, 512, 4224), (33, 512, 2176)]
 # the 96x192 ring tile: ragged tokens with an odd number of K blocks, K shorter than the ring (2 and 1 blocks),
 # 65 tokens (its lower bound)
 RING_SHAPES = [(100, 24576, 640), (150, 24576, 256), (192, 24576, 128), (65, 24576, 1024)]
@@ -285,7 +288,8 @@ def test_skinny_gemm_split_repeatable_and_without_workspace():
 
 
 @pytest.mark.parametrize("M,N,K,out_dtype", [(192, 6144, 4096, torch.bfloat16), (256, 2048, 4096, torch.float16),
-                                             (33, 1024, 2048, torch.bfloat16)])
+                                             (33, 1024, 2048, torch.bfloat16), (256, 2048, 6144, torch.float16),
+                                             (33, 1024, 3072, torch.bfloat16)])
 def test_skinny_gemm_matches_oracle(M, N, K, out_dtype):
     """Random codes and scales over five decades (two for fp16 outputs) on the
     small-M kernel, against the oracle's accumulator."""
@@ -366,14 +370,18 @@ def test_act_quant_edge_groups(dtype):
     assert np.array_equal(_bits(xs), xs_ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(4001, 4096, 128), (4096, 4096, 256), (3850, 4096, 384), (8000, 2048, 1152),
-                                   (1889, 4096, 128), (1900, 4096, 256), (2048, 4096, 384), (1800, 4096, 512),
-                                   (1793, 4096, 1152)])
-def test_group_swap_tiles(M, N, K):
+@pytest.mark.parametrize("kernel,M,N,K", [
+    (1, 4001, 4096, 128), (1, 4096, 4096, 256), (1, 3850, 4096, 384), (0, 8000, 2048, 1152), (1, 1889, 4096, 128),
+    (1, 1900, 4096, 256), (1, 2048, 4096, 384), (1, 1800, 4096, 512), (1, 1793, 4096, 1152),
+    (0, 2017, 24576, 384), (0, 3850, 4096, 512), (0, 3481, 4096, 640), (0, 1346, 8192, 1152), (0, 1773, 6144, 1280),
+    (5, 126, 51200, 1152), (5, 980, 8192, 1280), (5, 249, 24576, 1408), (5, 65, 51200, 1536), (5, 1793, 4096, 1664)])
+def test_group_swap_tiles(kernel, M, N, K):
     """The 256 x 256 and 256 x 128 tiles whose two wave groups take turns, from
-    one K block (the prologue's loads only) over the ring's depth to more,
-    with a ragged last tile; against the block-scaled sum in torch fp32."""
+    the fewest K blocks that are given to them (3 and 9: every phase of the two
+    and three buffers) on, and the calls of 128 x 64 tiles beside them; ragged
+    last tiles.  Against the block-scaled sum in torch fp32."""
     announce(f"fp8 linear: GEMM {M} x {N} x {K}, wave groups in turn")
+    assert _native.load().nvamd_fp8_linear_kernel(M, N, K, 1, None) == kernel
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     xq = torch.randint(0, 256, (M, K), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
     w = torch.randint(0, 256, (N, K), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
@@ -393,8 +401,9 @@ def test_group_swap_tiles(M, N, K):
     assert not bad.any(), f"{int(bad.sum())} outputs off, first at {bad.nonzero()[0].tolist()}"
 
 
-@pytest.mark.parametrize("kernel,M,N,K", [(0, 3851, 4096, 384), (5, 1793, 4096, 1152), (1, 1001, 2048, 512),
-                                          (4, 100, 24576, 640), (6, 77, 2048, 2176), (7, 9, 512, 1152)])
+@pytest.mark.parametrize("kernel,M,N,K", [(0, 3851, 4096, 512), (5, 249, 24576, 1408), (1, 1001, 2048, 512),
+                                          (3, 77, 2048, 1664), (4, 100, 24576, 640), (6, 77, 2048, 2688),
+                                          (7, 9, 512, 1152)])
 def test_weights_in_the_last_columns_of_a_wider_matrix(kernel, M, N, K):
     """Weights that are the last K columns of a matrix with longer rows: the
     last row ends with the matrix, so no kernel may read past its K bytes (the
