@@ -123,6 +123,18 @@ __host__ __device__ constexpr int64_t round_up_1k(int64_t b) { return (b + 1023)
 __device__ __forceinline__ uint32_t x_bytes(const Fp8GemmParams& p, int rows) {
   return (uint32_t)(rows - 1) * p.x_row + (uint32_t)(p.Kc - 1) * p.x_blk + (uint32_t)kFp8Block;
 }
+// Descriptor of K block kc (< p.Kc; past it an empty one) of `rows` token rows
+// from row m0 on, rows p.x_row apart: it ends with the last row's 128 bytes,
+// so rows past it read zeros in either layout and cost no traffic.  With the
+// activations by K block one descriptor for all blocks lets them read the next
+// block's rows (65 tokens on the 96 x 192 tile, 24,576 x 4,096: 33.3 us, 31.7
+// with this; 12 on 128 x 64, 51,200 x 5,120: 64.5, 59.7), which is cheaper
+// where a tile has few rows (64 x 16, 1,024 x 4,096 at 640 tokens: 21.0, 21.5
+// with this): tiles of 64 tokens and more use this one.
+__device__ __forceinline__ u32x4 x_block_rsrc(const Fp8GemmParams& p, int64_t m0, int rows, int kc) {
+  return rsrc_words(p.xq + m0 * p.x_row + (int64_t)kc * p.x_blk,
+                    kc < p.Kc ? (uint32_t)(rows - 1) * p.x_row + (uint32_t)kFp8Block : 0u);
+}
 __device__ __forceinline__ uint32_t sx_bytes(const Fp8GemmParams& p, int rows) {
   return (((uint32_t)(rows - 1) * p.sx_row + (uint32_t)(p.Kc - 1) * p.sx_blk + 1u) * 2u + 3u) & ~3u;
 }
@@ -174,10 +186,11 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
   const int Kc = p.Kc;
   const int rows_x = (int)min((int64_t)T::BM, p.M - m0);  // valid token rows of the tile
 
-  // descriptors: rows past the matrix (tokens >= M) read zeros or, with the
-  // activations by K block, the next block's rows (their columns are not stored)
+  // descriptors: rows past the matrix (tokens >= M) read zeros or, in small
+  // tiles, the next block's rows (their columns are not stored)
   const u32x4 rw = rsrc_words(p.w + (int64_t)n0 * p.w_stride, (uint32_t)((int64_t)T::BN * p.w_stride));
   const u32x4 rx = rsrc_words(p.xq + m0 * p.x_row, x_bytes(p, rows_x));
+  constexpr bool kBlockRsrc = T::BM >= 64;  // see x_block_rsrc
   const u32x4 rsx = rsrc_words(p.x_scale + m0 * p.sx_row, sx_bytes(p, rows_x));
   // weight scales from a 16-byte aligned element (sw_shift elements before the tile's first)
   const int64_t sw_first = (int64_t)(n0 / kFp8Block) * Kc;
@@ -197,7 +210,7 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
   };
   auto x_off = [&](int i, int kc) {
     const int r = 8 * (wave + T::kWaves * i) + fr;
-    return (uint32_t)r * p.x_row + (uint32_t)kc * p.x_blk + (uint32_t)(16 * (fp ^ frag_swz(r)));
+    return (uint32_t)r * p.x_row + (kBlockRsrc ? 0u : (uint32_t)kc * p.x_blk) + (uint32_t)(16 * (fp ^ frag_swz(r)));
   };
   // wave w < kSxLoads: token rows 64 w + lane, the dword holding x_scale[row][kc]
   const uint32_t sx_row_off = (uint32_t)(64 * wave + lane) * p.sx_row * 2u;
@@ -211,9 +224,10 @@ __global__ __launch_bounds__(64 * WN * WM) void block_gemm_kernel(Fp8GemmParams 
       if constexpr (S > 2) dma_load16(rw, w_off(i, kc), base + (uint32_t)(1024 * (wave + T::kWaves * i)));
       else dma_load16_keep(rw, w_off(i, kc), base + (uint32_t)(1024 * (wave + T::kWaves * i)));
     }
+    const u32x4 rxk = kBlockRsrc ? x_block_rsrc(p, m0, rows_x, kc) : rx;
 #pragma unroll
     for (int i = 0; i < T::kXLoads; ++i)
-      dma_load16_keep(rx, x_off(i, kc), base + (uint32_t)(T::kWBytes + 1024 * (wave + T::kWaves * i)));
+      dma_load16_keep(rxk, x_off(i, kc), base + (uint32_t)(T::kWBytes + 1024 * (wave + T::kWaves * i)));
     if (wave < T::kSxLoads)
       dma_load4_keep(rsx, (sx_row_off + 2u * p.sx_blk * (uint32_t)kc) & ~3u, base + (uint32_t)(T::kWBytes + T::kXBytes + 256 * wave));
   };
@@ -660,7 +674,6 @@ __global__ __launch_bounds__((64 * Skinny<CW, MF>::kWaves)) void skinny_gemm_ker
   if (wave >= CW) {
     // ---- loader waves ------------------------------------------------------
     const int l = wave - CW;
-    const u32x4 rx = rsrc_words(p.xq, x_bytes(p, (int)p.M));
     const u32x4 rsx = rsrc_words(p.x_scale, sx_bytes(p, (int)p.M));
     if (l == 0) {
       const u32x4 rsw = rsrc_words(p.w_scale + (sw_first - sw_shift), (uint32_t)(((int64_t)nk + sw_shift) * 2 + 3) & ~3u);
@@ -672,12 +685,12 @@ __global__ __launch_bounds__((64 * Skinny<CW, MF>::kWaves)) void skinny_gemm_ker
     // bytes are never read), so every wait below counts the same loads.
     auto issue_stage = [&](int kc, int s) {
       const uint32_t base = lds0 + (uint32_t)(s * T::kStage);
+      const u32x4 rx = x_block_rsrc(p, 0, (int)p.M, kc);
 #pragma unroll
       for (int i0 = 0; i0 < T::kXLoads; i0 += T::LW) {
         const int i = i0 + l;
         const int r = 8 * i + fr;
-        dma_load16_keep(rx, (uint32_t)r * p.x_row + (uint32_t)kc * p.x_blk + 16u * (uint32_t)(fp ^ frag_swz(r)),
-                        base + 1024u * i);
+        dma_load16_keep(rx, (uint32_t)r * p.x_row + 16u * (uint32_t)(fp ^ frag_swz(r)), base + 1024u * i);
       }
       if (l == 0) {
 #pragma unroll
