@@ -70,24 +70,37 @@ int32_t noalloc_scratch(const char* fn, void** out) {
   return NVAMD_OK;
 }
 
-// CUs of the current device, looked up once per device (every host call
-// sizes its grid and workspace from it).
-std::atomic<int> g_cu_count[kMaxDevices];
+// CUs of the current device and the LDS of one workgroup on it, looked up once
+// per device (every host call sizes its grid and workspace from them).  No
+// device: an MI355X's.
+struct DeviceLimits {
+  int cus = 256, lds = 160 * 1024;
+};
+std::atomic<int64_t> g_limits[kMaxDevices];  // cus << 32 | lds, 0: not looked up yet
 
-int device_cu_count() {
+DeviceLimits device_limits() {
+  DeviceLimits d;
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (hipGetDevice(&dev) != hipSuccess) return d;
   const bool cached = dev >= 0 && dev < kMaxDevices;
   if (cached) {
-    const int n = g_cu_count[dev].load(std::memory_order_relaxed);
-    if (n > 0) return n;
+    const int64_t v = g_limits[dev].load(std::memory_order_relaxed);
+    if (v != 0) {
+      d.cus = (int)(v >> 32);
+      d.lds = (int)(v & 0x7fffffff);
+      return d;
+    }
   }
-  int cus = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  if (cached) g_cu_count[dev].store(cus, std::memory_order_relaxed);
-  return cus;
+  int cus = 0, lds = 0;
+  const bool got_cus = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0;
+  const bool got_lds = hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && lds > 0;
+  if (got_cus) d.cus = cus;
+  if (got_lds) d.lds = lds;
+  if (cached && got_cus && got_lds) g_limits[dev].store((int64_t)d.cus << 32 | d.lds, std::memory_order_relaxed);
+  return d;
 }
+
+int device_cu_count() { return device_limits().cus; }
 
 constexpr int kHeadDim = 128;
 
@@ -219,6 +232,34 @@ PrefillLayout prefill_layout(int32_t num_seqs, int32_t num_kv_heads, int g, int3
   return L;
 }
 
+// The kernel of a product on the current device, planned once per call
+// (raw_x: by the whole layer, which may quantise in the kernel).
+struct LinearPlan {
+  nvamd::ThinPlan thin;      // mf > 0: the kernel for few tokens
+  nvamd::SkinnyPlan skinny;  // else cw > 0: the small-M kernel
+  int config = -1;           // else this tile (-1: no tile's scales fit the LDS)
+};
+
+LinearPlan plan_linear(int64_t M, int64_t N, int Kc, bool raw_x, int64_t workspace_bytes) {
+  const DeviceLimits d = device_limits();
+  LinearPlan pl;
+  pl.thin = nvamd::fp8_thin_plan(M, N, Kc, d.cus, d.lds, raw_x);
+  if (pl.thin.mf > 0) return pl;
+  pl.skinny = nvamd::fp8_skinny_plan(M, N, Kc, d.cus, workspace_bytes, d.lds);
+  if (pl.skinny.cw > 0) return pl;
+  pl.config = nvamd::fp8_gemm_pick_config(M, N, Kc, d.cus, d.lds);
+  return pl;
+}
+
+bool linear_sizes(int64_t M, int64_t N, int64_t K) {
+  return M > 0 && N > 0 && K > 0 && N % 128 == 0 && K % 128 == 0 && N <= 0x7fffffffll && K <= 0x7fffffffll;
+}
+
+// Workspace of the small-M kernel's partial sums (0: another kernel, or K whole).
+int64_t split_bytes(const LinearPlan& pl, int64_t M, int64_t N) {
+  return pl.skinny.splits > 1 ? (int64_t)pl.skinny.splits * M * N * 4 : 0;
+}
+
 }  // namespace
 
 extern "C" {
@@ -320,21 +361,9 @@ int32_t nvamd_fp8_act_quant(const void* x, int64_t x_stride0, int32_t x_dtype, v
                        fn);
 }
 
-namespace {
-
-int64_t device_lds_limit() {
-  int dev = 0, lds_limit = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || lds_limit <= 0)
-    lds_limit = 160 * 1024;
-  return lds_limit;
-}
-
-}  // namespace
-
 int64_t nvamd_fp8_block_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > 0x7fffffffll || K > 0x7fffffffll) return 0;
-  return nvamd::fp8_skinny_workspace_bytes(M, N, (int)(K / 128), device_cu_count(), device_lds_limit());
+  if (!linear_sizes(M, N, K) || M > nvamd::kSkinnyMaxM) return 0;
+  return split_bytes(plan_linear(M, N, (int)(K / 128), false, INT64_MAX), M, N);
 }
 
 namespace {
@@ -390,21 +419,21 @@ nvamd::Fp8GemmParams gemm_params(const void* xq, const void* x_scale, const void
   return p;
 }
 
-// The GEMM on quantised activations: the kernel its sizes call for.
-int32_t run_block_gemm(const char* fn, const nvamd::Fp8GemmParams& p, bool f16_out, void* workspace,
-                       int64_t workspace_bytes, hipStream_t stream) {
-  const int64_t lds_limit = device_lds_limit();
-  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(p.M, p.N, p.Kc, device_cu_count(), lds_limit, false);
-  if (thin.mf > 0)
-    return launch_status(nvamd::launch_fp8_thin_linear(p, thin, nullptr, 0, false, f16_out, stream), fn);
-  const nvamd::SkinnyPlan plan = nvamd::fp8_skinny_plan(p.M, p.N, p.Kc, device_cu_count(), workspace_bytes, lds_limit);
-  if (plan.cw > 0)
-    return launch_status(nvamd::launch_fp8_skinny_gemm(p, plan, f16_out, static_cast<float*>(workspace), stream), fn);
-  const int config = nvamd::fp8_gemm_pick_config(p.M, p.N, p.Kc, device_cu_count(), lds_limit);
-  if (config < 0)
-    return fail(NVAMD_ERR_UNSUPPORTED, "%s: K=%lld needs more LDS for the tile scales than the device has", fn,
-                (long long)p.K);
-  return launch_status(nvamd::launch_fp8_block_gemm(p, config, f16_out, stream), fn);
+// The planned GEMM on quantised activations.
+int32_t run_block_gemm(const char* fn, const nvamd::Fp8GemmParams& p, const LinearPlan& pl, bool f16_out,
+                       void* workspace, hipStream_t stream) {
+  if (pl.thin.mf > 0)
+    return launch_status(nvamd::launch_fp8_thin_linear(p, pl.thin, nullptr, 0, false, f16_out, stream), fn);
+  if (pl.skinny.cw > 0)
+    return launch_status(nvamd::launch_fp8_skinny_gemm(p, pl.skinny, f16_out, static_cast<float*>(workspace), stream),
+                         fn);
+  return launch_status(nvamd::launch_fp8_block_gemm(p, pl.config, f16_out, stream), fn);
+}
+
+int32_t no_plan(const char* fn, const LinearPlan& pl, int64_t K) {
+  if (pl.thin.mf > 0 || pl.skinny.cw > 0 || pl.config >= 0) return NVAMD_OK;
+  return fail(NVAMD_ERR_UNSUPPORTED, "%s: K=%lld needs more LDS for the tile scales than the device has", fn,
+              (long long)K);
 }
 
 // nvamd_fp8_block_linear's scratch: the quantised activations and their
@@ -423,34 +452,31 @@ int32_t nvamd_fp8_block_gemm(const void* xq, const void* x_scale, const void* we
   if (M == 0) return ok();
   if (!x_scale) return fail(NVAMD_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
   if ((uintptr_t)x_scale % 16 != 0) return fail(NVAMD_ERR_UNSUPPORTED, "%s: operands must be 16-byte aligned", fn);
+  const LinearPlan pl = plan_linear(M, N, (int)(K / 128), false, workspace_bytes);
+  if (int32_t e = no_plan(fn, pl, K)) return e;
   return run_block_gemm(fn, gemm_params(xq, x_scale, weight, weight_stride0, weight_scale, out, out_stride0, M, N, K),
-                        out_dtype == NVAMD_DTYPE_F16, workspace, workspace_bytes, (hipStream_t)stream);
+                        pl, out_dtype == NVAMD_DTYPE_F16, workspace, (hipStream_t)stream);
 }
 
 int32_t nvamd_fp8_linear_kernel(int64_t M, int64_t N, int64_t K, int32_t quantised, int64_t* lds_bytes) {
   if (lds_bytes) *lds_bytes = 0;
-  if (M <= 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > 0x7fffffffll || K > 0x7fffffffll) return -1;
-  const int Kc = (int)(K / 128), cus = device_cu_count();
-  const int64_t lds_limit = device_lds_limit();
-  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(M, N, Kc, cus, lds_limit, quantised == 0);
-  if (thin.mf > 0) {
-    if (lds_bytes) *lds_bytes = thin.lds;
-    return thin.xi > 0 ? NVAMD_LINEAR_FEW_TOKENS_X : NVAMD_LINEAR_FEW_TOKENS;
-  }
-  const nvamd::SkinnyPlan plan = nvamd::fp8_skinny_plan(M, N, Kc, cus, INT64_MAX, lds_limit);
-  if (plan.cw > 0) {
-    if (lds_bytes) *lds_bytes = nvamd::fp8_skinny_lds_bytes(plan);
-    return NVAMD_LINEAR_SMALL_M;
-  }
-  const int config = nvamd::fp8_gemm_pick_config(M, N, Kc, cus, lds_limit);
-  if (config >= 0 && lds_bytes) *lds_bytes = nvamd::fp8_gemm_lds_bytes(config, Kc);
-  return config;
+  if (!linear_sizes(M, N, K)) return -1;
+  const int Kc = (int)(K / 128);
+  const LinearPlan pl = plan_linear(M, N, Kc, quantised == 0, INT64_MAX);
+  const int64_t lds = pl.thin.mf > 0      ? pl.thin.lds
+                      : pl.skinny.cw > 0  ? nvamd::fp8_skinny_lds_bytes(pl.skinny)
+                      : pl.config >= 0    ? nvamd::fp8_gemm_lds_bytes(pl.config, Kc)
+                                          : 0;
+  if (lds_bytes) *lds_bytes = lds;
+  if (pl.thin.mf > 0) return pl.thin.xi > 0 ? NVAMD_LINEAR_FEW_TOKENS_X : NVAMD_LINEAR_FEW_TOKENS;
+  return pl.skinny.cw > 0 ? NVAMD_LINEAR_SMALL_M : pl.config;
 }
 
 int64_t nvamd_fp8_block_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || N > 0x7fffffffll || K > 0x7fffffffll) return 0;
-  if (nvamd::fp8_thin_plan(M, N, (int)(K / 128), device_cu_count(), device_lds_limit(), true).xi > 0) return 0;
-  return act_bytes(M, K) + nvamd_fp8_block_gemm_workspace_bytes(M, N, K);
+  if (!linear_sizes(M, N, K)) return 0;
+  if (M > nvamd::kSkinnyMaxM) return act_bytes(M, K);  // a tile, whichever
+  const LinearPlan pl = plan_linear(M, N, (int)(K / 128), true, INT64_MAX);
+  return pl.thin.xi > 0 ? 0 : act_bytes(M, K) + split_bytes(pl, M, N);
 }
 
 int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype, const void* weight,
@@ -466,12 +492,13 @@ int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype
   const bool f16 = x_dtype == NVAMD_DTYPE_F16;
   nvamd::Fp8GemmParams p =
       gemm_params(nullptr, nullptr, weight, weight_stride0, weight_scale, out, out_stride0, M, N, K);
-  const nvamd::ThinPlan thin = nvamd::fp8_thin_plan(M, N, p.Kc, device_cu_count(), device_lds_limit(), true);
-  if (thin.xi > 0)
-    return launch_status(nvamd::launch_fp8_thin_linear(p, thin, x, x_stride0, f16, f16, (hipStream_t)stream), fn);
-  const int64_t act = act_bytes(M, K);
+  const int64_t act = act_bytes(M, K), left = std::max<int64_t>(workspace_bytes - act, 0);
+  const LinearPlan pl = plan_linear(M, N, p.Kc, true, left);
+  if (pl.thin.xi > 0)
+    return launch_status(nvamd::launch_fp8_thin_linear(p, pl.thin, x, x_stride0, f16, f16, (hipStream_t)stream), fn);
   if (workspace_bytes < act)
     return fail(NVAMD_ERR_WORKSPACE, "%s: workspace of %lld bytes needed", fn, (long long)act);
+  if (int32_t e = no_plan(fn, pl, K)) return e;
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   p.xq = ws;
   p.x_scale = reinterpret_cast<const uint16_t*>(ws + align_up(M * K));
@@ -487,8 +514,7 @@ int32_t nvamd_fp8_block_linear(const void* x, int64_t x_stride0, int32_t x_dtype
   } else if (int32_t e = nvamd_fp8_act_quant(x, x_stride0, x_dtype, ws, ws + align_up(M * K), M, K, stream)) {
     return e;
   }
-  const int64_t left = workspace_bytes - act;
-  return run_block_gemm(fn, p, f16, left > 0 ? ws + act : nullptr, left, (hipStream_t)stream);
+  return run_block_gemm(fn, p, pl, f16, left > 0 ? ws + act : nullptr, (hipStream_t)stream);
 }
 
 int32_t nvamd_build_attention_metadata(const int32_t* packed, int64_t packed_ints, int32_t num_seqs, int32_t num_plain,

@@ -991,11 +991,6 @@ SkinnyPlan fp8_skinny_plan(int64_t M, int64_t N, int Kc, int cus, int64_t worksp
   return best;
 }
 
-int64_t fp8_skinny_workspace_bytes(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit) {
-  const SkinnyPlan pl = fp8_skinny_plan(M, N, Kc, cus, INT64_MAX, lds_limit);
-  return pl.cw > 0 && pl.splits > 1 ? (int64_t)pl.splits * M * N * 4 : 0;
-}
-
 int64_t fp8_skinny_lds_bytes(const SkinnyPlan& plan) { return skinny_lds(plan.cw, plan.mf, plan.kper); }
 
 hipError_t launch_fp8_skinny_gemm(const Fp8GemmParams& p, const SkinnyPlan& plan, bool f16_out, float* part,

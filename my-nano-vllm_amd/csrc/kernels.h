@@ -170,7 +170,6 @@ struct SkinnyPlan {
   int cw = 0, mf = 0, splits = 1, kper = 0;
 };
 SkinnyPlan fp8_skinny_plan(int64_t M, int64_t N, int Kc, int cus, int64_t workspace_bytes, int64_t lds_limit);
-int64_t fp8_skinny_workspace_bytes(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit);
 int64_t fp8_skinny_lds_bytes(const SkinnyPlan& plan);
 hipError_t launch_fp8_skinny_gemm(const Fp8GemmParams& p, const SkinnyPlan& plan, bool f16_out, float* part,
                                   hipStream_t stream);
