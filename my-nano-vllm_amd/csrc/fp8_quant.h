@@ -21,10 +21,14 @@ __device__ __forceinline__ float in_to_f32(uint32_t bits16) {
 //
 // The division is the cost of this step, so x / scale is taken as a product
 // with the group's reciprocal r = RN(1 / scale) and one correction,
-// q = x r, q - (q scale - x) r with the remainder exact (and signed so that -0
-// stays -0): the correctly rounded quotient, as long as nothing leaves the normal range (checked exhaustively
-// over the significands of bf16 and fp16 x and amax).  A group with a
-// non-finite value or a scale outside 2^+-100 takes the divisions instead.
+// q = x r, q - (q scale - x) r (signed so that -0 stays -0).  The remainder is
+// exact where q scale has no bits below 2^-149, and the result is then the
+// correctly rounded quotient; at the smallest scales the remainder of a
+// quotient below 1 loses its last bits, which can move a result that lies
+// halfway between two fp32 values, not its E4M3 byte.  The bytes equal those of
+// the division for every pair of significands of x and amax, in bf16 and fp16,
+// at scales of both ends of the range too (a test).  A group with a non-finite
+// value or a scale outside 2^+-100 takes the divisions instead.
 template <bool F16_IN>
 __device__ __forceinline__ u32x2 quant_group8(u32x4 w, float& scale) {
   const uint32_t d[4] = {w.x, w.y, w.z, w.w};

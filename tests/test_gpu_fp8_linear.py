@@ -448,3 +448,87 @@ def test_infinite_weight_scale_in_the_last_block(M, N, K):
     want[:, 5] = -float("inf")
     assert torch.equal(got[:, :128], want), got[:, :8]
     assert torch.isfinite(got[:, 128:]).all()
+
+
+@pytest.mark.parametrize("kernel,M,N,K", [
+    (0, 3481, 4096, 640), (0, 2017, 24576, 384), (1, 1001, 2048, 512), (2, 1000, 1024, 128), (3, 301, 128, 256),
+    (3, 77, 2048, 1664), (4, 191, 24576, 640), (4, 67, 24576, 384), (5, 249, 24576, 1408), (5, 1793, 4096, 1664),
+    (6, 77, 2048, 2688), (6, 191, 4096, 12288), (6, 255, 1024, 6272), (6, 33, 512, 4224), (7, 9, 512, 1152),
+    (7, 31, 4096, 1024)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_layer_equals_its_two_steps(kernel, M, N, K, dtype):
+    """The layer quantises into a layout by K block ([K/128, M, 128] and
+    [K/128, M]), the two C entry points by row ([M, K] and [M, K/128]): the
+    same kernel on the same numbers in the same order, so the same bits; on
+    every kernel, with odd token counts (a scale is then either half of its
+    dword from block to block) and ragged last tiles (their rows past M would
+    be the next block's)."""
+    announce(f"fp8 linear: layer against its two steps, {M} x {N} x {K} {dtype}")
+    lib = _native.load()
+    assert lib.nvamd_fp8_linear_kernel(M, N, K, 0, None) == kernel
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = (torch.randn(M, K, generator=g, device="cuda") * 3).to(dtype)
+    x *= 10.0 ** torch.empty(M, 1, device="cuda").uniform_(-1, 1, generator=g)
+    w = torch.randint(0, 256, (N, K), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    w = torch.where((w & 0x7F) == 0x7F, w ^ 0x01, w)
+    w_scale = (torch.rand(N // 128, K // 128, generator=g, device="cuda") * 2e-4 + 1e-4).to(torch.bfloat16)
+    got = fp8_block_linear(x, w.view(torch.float8_e4m3fn), w_scale)
+    xq = torch.empty(M, K, dtype=torch.uint8, device="cuda")
+    xs = torch.empty(M, K // 128, dtype=torch.bfloat16, device="cuda")
+    _native.check(lib.nvamd_fp8_act_quant(x.data_ptr(), K, 0 if dtype == torch.bfloat16 else 1, xq.data_ptr(),
+                                          xs.data_ptr(), M, K, torch.cuda.current_stream().cuda_stream), "act_quant")
+    want = _gemm_gpu(xq, xs, w, w_scale, dtype)
+    assert torch.isfinite(want.float()).all() and float(want.float().abs().max()) > 0
+    assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16))
+
+
+def test_layer_beyond_32_bit_block_offsets():
+    """2^31 quantised bytes and more: the layer keeps its activations by row.
+    Its first and last rows have the bits of the same rows in a call of their
+    own (by K block; every tile adds the blocks in the same order)."""
+    M, N, K = (1 << 19) + 77, 128, 4096
+    announce(f"fp8 linear: layer of {M} x {K} activations, by row")
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.empty(M, K, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    w = torch.randint(0, 120, (N, K), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    w, w_scale = w.view(torch.float8_e4m3fn), torch.full((1, K // 128), 1e-3, dtype=torch.bfloat16, device="cuda")
+    got = fp8_block_linear(x, w, w_scale)
+    for rows in (slice(0, 4096), slice(M - 4099, M)):
+        assert torch.equal(got[rows].view(torch.int16), fp8_block_linear(x[rows], w, w_scale).view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_act_quant_every_significand_pair(dtype):
+    """The quantisation's division as a product with the reciprocal and one
+    correction: every significand of the group's maximum against every
+    significand of a value beside it, from the maximum's binade down to below
+    half of the smallest E4M3 value; in bf16 also with scales next to 2^-100
+    and 2^100, the ends of its range.  Codes and scales equal the oracle's IEEE
+    divisions."""
+    announce(f"fp8 linear: activation quant, every pair of significands {dtype}")
+    bits = 7 if dtype == torch.bfloat16 else 10
+    sig = 1.0 + torch.arange(2 ** bits, dtype=torch.float64) / 2 ** bits
+    tops = [13] if dtype == torch.float16 else [0, -93, -92, 107]  # scales from 2^(top - 7.8) to 2^(top - 6.8)
+    for top in tops:
+        down = sig[None, :] * 2.0 ** (top - torch.arange(0, 21, dtype=torch.float64))[:, None]
+        values = down.reshape(-1)                                          # 21 binades x all significands
+        groups = -(-len(values) // 127)
+        padded = torch.zeros(groups * 127, dtype=torch.float64)
+        padded[:len(values)] = values
+        for maxima in (sig * 2.0 ** (top + 1)).split(256):
+            x = torch.empty(len(maxima), groups, 128, dtype=torch.float64)
+            x[:, :, 1:] = padded.view(1, groups, 127)
+            x[:, :, 0] = maxima[:, None]
+            x[:, 1::2] *= -1.0
+            x = x.reshape(len(maxima), groups * 128).to(dtype)
+            xq_ref, xs_ref, _ = ol.act_quant(x)
+            lib = _native.load()
+            M, K = x.shape
+            xd = x.cuda()
+            xq = torch.empty(M, K, dtype=torch.uint8, device="cuda")
+            xs = torch.empty(M, K // 128, dtype=torch.bfloat16, device="cuda")
+            _native.check(lib.nvamd_fp8_act_quant(xd.data_ptr(), K, 0 if dtype == torch.bfloat16 else 1, xq.data_ptr(),
+                                                  xs.data_ptr(), M, K, torch.cuda.current_stream().cuda_stream), "quant")
+            torch.cuda.synchronize()
+            assert np.array_equal(xq.cpu().numpy(), xq_ref)
+            assert np.array_equal(_bits(xs), xs_ref)
