@@ -950,15 +950,15 @@ SkinnyPlan fp8_skinny_plan(int64_t M, int64_t N, int Kc, int cus, int64_t worksp
   // Where the tile kernels are faster (GPU time of both sides on 41 shapes of K
   // 128 to 32,768 and N 128 to 51,200; profiles/fp8_linear_kernels.md):
   //  - their grid covers the CUs, with 64-feature tiles for 64 tokens too (us
-  //    per call, tiles / this kernel: 64 tokens on 24,576 x 4,096 34.2 / 40.1,
-  //    on 19,456 x 2,560 22.9 / 33.9; but on 10,240 x 5,120 32.4 / 28.3);
+  //    per call, tiles / this kernel: 64 tokens on 24,576 x 4,096 31.6 / 39.6,
+  //    on 19,456 x 2,560 22.8 / 33.4; but on 10,240 x 5,120 32.4 / 28.1);
   //  - short rows, where a K split has little to share out.  The tiles' time is
   //    one K block after another whatever M is, this kernel's grows with M, so
-  //    the line moves up with it: 64 tokens on 1,024 x 2,048 10.6 / 10.4 (and a
-  //    launch fewer), on 1,024 x 3,072 13.7 / 10.9; 128 on 1,024 x 2,048 10.7 /
-  //    12.8, on 6,144 x 2,560 18.4 / 18.9, on 1,024 x 4,096 16.8 / 14.2; 192 on
-  //    5,120 x 3,200 22.1 / 29.1, on 1,024 x 4,096 17.5 / 15.9; 256 on 4,096 x
-  //    4,096 26.5 / 28.1, on 1,024 x 6,144 24.8 / 21.3.
+  //    the line moves up with it: 64 tokens on 1,024 x 2,048 10.6 / 10.2 (and a
+  //    launch fewer), on 1,024 x 3,072 13.6 / 10.6; 128 on 1,024 x 2,048 10.7 /
+  //    12.0, on 6,144 x 2,560 18.5 / 18.2, on 1,024 x 4,096 16.8 / 13.5; 192 on
+  //    5,120 x 3,200 22.2 / 29.3, on 1,024 x 4,096 17.3 / 15.9; 224 on 4,096 x
+  //    4,096 26.9 / 28.3, 256 on 1,024 x 6,144 24.8 / 21.2.
   if ((N / 128) * ((M + 63) / 64) >= cus || N / 64 >= cus) return best;
   if (Kc <= (M <= 32 ? 5 : M <= 64 ? 16 : M <= 128 ? 20 : M <= 192 ? 25 : 40)) return best;
   const int mf = M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : M <= 128 ? 8 : M <= 192 ? 12 : 16;
@@ -1027,10 +1027,10 @@ hipError_t launch_fp8_act_quant(const void* x, int64_t x_stride, bool f16_in, vo
 // is within 0.3 % of the fastest in the mean).  A CU takes one large tile at a
 // time, 1.75 (256 x 256) or 1.15 (256 x 128) us per K block with all CUs busy
 // and 1.3 or 0.95 with few, and 6 or 5 us to fill and drain each (6,144 x 1,024
-// at 1,536 tokens: 30.2 on 256 x 256, 26.0 on 128 x 64); 128 x 64 tiles share a
+// at 1,536 tokens: 30.2 on 256 x 256, 25.9 on 128 x 64); 128 x 64 tiles share a
 // CU, 0.4 us per K block each.  Rows of tiles that cover more than half of the
 // CUs run one after another and read weights beyond the L2 again each (51,200 x
-// 5,120 at 257 tokens: 193 us on 128 x 64, 149 on 256 x 256).
+// 5,120 at 257 tokens: 192 us on 128 x 64, 148 on 256 x 256).
 static double gemm_estimate(int config, int64_t M, int64_t N, int Kc, int cus) {
   const int64_t rows = (M + kGemmBM[config] - 1) / kGemmBM[config];
   const double x = (double)(N / kGemmBN[config] * rows) / cus;
@@ -1051,13 +1051,13 @@ int fp8_gemm_pick_config(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limi
   auto tiles = [&](int c) { return (N / kGemmBN[c]) * ((M + kGemmBM[c] - 1) / kGemmBM[c]); };
   auto fits = [&](int c) { return N % kGemmBN[c] == 0 && config_lds_bytes(c, Kc) <= lds_limit; };
   // 32 < M <= 192 with whole 96-feature tiles covering the CUs (24,576 x
-  // 4,096, us per call: 48 tokens 29.9 against 36.5 on 128 x 64 tiles, 192
-  // tokens 40.2 against 46.6)
+  // 4,096, us per call: 48 tokens 31.2 against 36.5 on 128 x 64 tiles, 192
+  // tokens 38.6 against 45.5)
   if (M > 32 && M <= kGemmBM[4] && fits(4) && N / kGemmBN[4] >= cus) return 4;
   // Enough 128 x 64 tiles for the CUs: the fastest of the three large tiles
   // by the estimate (us per call; 256 x 256 / 256 x 128 / 128 x 64):
-  // 24,576 x 4,096, M 512: 62.0 / 81.6 / 90.6; 4,096 x 12,288, M 1,888: 146 /
-  // 124 / 162; 4,096 x 4,096, M 1,024: 54.1 / 39.1 / 29.3.
+  // 24,576 x 4,096, M 512: 66.6 / 85.0 / 90.7; 4,096 x 12,288, M 1,792: 143 /
+  // 112 / 159; 4,096 x 4,096, M 1,024: 53.4 / 40.3 / 30.9.
   int best = -1;
   if (fits(1) && tiles(1) >= cus) {
     double best_t = 0.0;

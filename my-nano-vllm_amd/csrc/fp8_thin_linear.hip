@@ -231,23 +231,24 @@ hipError_t launch_thin(const Fp8GemmParams& p, const ThinPlan& pl, const void* x
 // fp8_linear.hip; more in profiles/fp8_linear_kernels.md).  Every workgroup
 // reads all the activations, so it loses its lead with M K (their bytes per
 // workgroup) and with M N (their reads in all):
-//   6,144 x 4,096:   M 1 7.7 / 16.5, 8 10.7 / 17.0, 16 12.3 / 17.4, 32 16.1 / 18.7
-//   24,576 x 4,096:  M 1 21.4 / 30.8, 16 29.8 / 31.6, 24 34.8 / 32.8, 32 38.9 / 33.3
-//   4,096 x 12,288:  M 1 13.1 / 20.9, 16 17.6 / 21.4, 24 20.6 / 22.1, 32 23.0 / 22.3
-//   5,120 x 25,600:  M 1 31.5 / 41.7, 8 40.1 / 42.1, 12 43.9 / 42.4, 16 47.6 / 42.4
-//   51,200 x 5,120:  M 1 47.6 / 56.3, 8 52.8 / 57.6, 12 56.8 / 57.8, 16 61.4 / 58.2
+//   6,144 x 4,096:   M 1 7.5 / 16.5, 8 10.5 / 17.2, 16 12.1 / 17.3, 32 15.9 / 18.4
+//   24,576 x 4,096:  M 1 21.1 / 30.6, 16 28.8 / 31.3, 24 35.4 / 33, 32 39.6 / 33
+//   4,096 x 12,288:  M 1 12.2 / 20.7, 16 17.2 / 21.4, 24 21.5 / 21.9, 32 23.6 / 22.1
+//   5,120 x 25,600:  M 1 30.3 / 41.8, 8 38.6 / 42.3, 12 42.0 / 42.5, 16 46.1 / 42.6
+//   51,200 x 5,120:  M 1 45.9 / 55.5, 8 51.8 / 56.8, 12 55.7 / 57.5, 16 60.6 / 57.9
 // With two workgroups on a CU a second token fragment doubles what the four
 // waves do per chunk:
-//   5,120 x 8,192:   M 16 18.7 / 20.0, 24 23.2 / 20.6
-//   6,144 x 1,024:   M 16 6.4 / 6.8, 24 7.5 / 7.0 (one wave per workgroup)
+//   5,120 x 8,192:   M 16 18.5 / 20.1, 24 23.2 / 21.2
+//   6,144 x 1,024:   M 16 6.3 / 6.8, 24 7.3 / 7.0 (one wave per workgroup)
 // Few workgroups leave CUs idle, which a K split would use: worth it only for
 // what one round of chunks holds.
-//   512 x 8,192:     M 1 6.3 / 10.0, 16 11.3 / 10.9, 32 14.9 / 11.1
-//   512 x 12,288:    M 1 8.7 / 11.1, 3 12.2 / 11.6, 16 13.8 / 11.9 (two rounds)
-//   256 x 32,768:    M 1 15.0 / 14.9, 3 22.4 / 15.1 (four rounds)
+//   512 x 8,192:     M 1 6.2 / 10.2, 16 10.9 / 11.1, 32 14.7 / 11.2
+//   512 x 12,288:    M 1 8.2 / 11.6, 3 11.9 / 11.8, 16 13.8 / 12.1 (two rounds)
+//   256 x 32,768:    M 1 14.3 / 15.2, 3 22.2 / 15.6 (four rounds)
 // Its own quantisation repeats per workgroup and pays for one or two tokens
-// (6,144 x 4,096, M = 2: 8.3 against 10.3; M = 4: 12.6 against 10.3), up to
-// four when every workgroup has a CU (4,096 x 4,096, M = 4: 7.9 against 10.3).
+// (6,144 x 4,096, M = 2: 8.2 against 9.9 with a launch before; M = 4: 12.6
+// against 9.9), up to four when every workgroup has a CU (4,096 x 4,096, M = 4:
+// 7.6, five tokens with a launch before 7.9).
 ThinPlan fp8_thin_plan(int64_t M, int64_t N, int Kc, int cus, int64_t lds_limit, bool raw_x) {
   ThinPlan pl;
   if (M < 1 || M > kThinMaxM || N % 128 != 0 || Kc < 1 || M * Kc > (1 << 11) || M * N > 600000) return pl;

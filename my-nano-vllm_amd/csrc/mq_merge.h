@@ -91,13 +91,14 @@ __host__ __device__ __forceinline__ int merge_slices(const MqParams& p, int n_wa
 
 // ---- balanced (stream-K) kernel: merge of a pair cut across workgroups ----
 
-// Workgroups that take stages, of a call with T stages: one stage each while
-// there are workgroups (T of them then share nothing but the merge), up to
-// one workgroup per CU; the rest of the grid (kernels of which a CU holds two
-// or three) from four stages each on.  A pair is cut into at most 64 ranges,
-// what the waves of the wide merge add in one round trip, unless those would
-// get more than four stages each.  us per call by workgroups (GPU time, 8 kv
-// heads, 32 query heads unless said otherwise; best of each):
+// Workgroups that take stages, of a call with T stages: as many as there are
+// stages, up to one per CU; the rest of the grid (kernels of which a CU holds
+// two or three) in whole multiples of the CUs, once fewer would leave more
+// than four stages each (608 workgroups on 256 CUs: 17.2 us where 512 and 768
+// take 15.1 and 15.6).  A pair is cut into at most 64 ranges, what the waves
+// of the wide merge add in one round trip, unless those would get more than
+// four stages each.  us per call by workgroups (GPU time, 32 query and 8 kv
+// heads unless said otherwise):
 //   1 x 777 tokens (49 stages)        49: 11.7, 24: 12.6
 //   1 x 2,048 (128)                   128: 13.4, 64: 12.8, 32: 14.0
 //   1 x 4,096 (256)                   256: 16.3, 128: 14.4, 64: 14.5
