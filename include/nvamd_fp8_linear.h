@@ -59,8 +59,8 @@ int32_t nvamd_fp8_act_quant(const void* x, int64_t x_stride0, int32_t x_dtype, v
  * tile's scales: NVAMD_ERR_UNSUPPORTED beyond it (K <= 32768 always fits).
  *
  * workspace (16-byte aligned, contents ignored; NULL with workspace_bytes 0
- * allowed): M <= 256 tokens take a kernel that streams each weight row once
- * and may split K over workgroups; it then writes fp32 partial sums there and
+ * allowed): at most 256 tokens may take a kernel that streams each weight row
+ * once and splits K over workgroups; it then writes fp32 partial sums there and
  * adds them in split order (repeated calls are bit-identical).  With less
  * than nvamd_fp8_block_gemm_workspace_bytes(M, N, K) bytes, K is split only
  * as far as the workspace holds.  The reference's launch has no workspace: its
